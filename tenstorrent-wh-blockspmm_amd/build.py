@@ -36,7 +36,7 @@ HIP_FLAGS = [
     "-Wall",
 ]
 
-SOURCES = ["bsp_kernels.hip", "bsp_capi.cpp", "bsp_schedule.cpp", "bsp_noalloc.hip"]
+SOURCES = ["bsp_kernels.hip", "bsp_tile.hip", "bsp_capi.cpp", "bsp_schedule.cpp", "bsp_noalloc.hip"]
 
 
 def _run(cmd: list[str]) -> str:

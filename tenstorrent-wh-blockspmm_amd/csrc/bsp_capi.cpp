@@ -40,6 +40,9 @@ struct bsp_plan {
     bsp::SpgemmRun* d_runs = nullptr;  // wave runs
     int32_t wg_per_xcd = 0;
     int32_t sddmm_one_shot = 0;  // SDDMM: the one-shot kernel runs this plan
+    int32_t tile = 0;            // SDDMM: the tile kernel runs this plan on tiles of that height
+    bsp::SddmmTileVariant sddmm_tile{};
+    int32_t cb_shift = 0;        // SDDMM tiles: log2 of the column chunks' width
     // SpMM persistent kernel: variant, unit records and A words (the B words
     // go in d_ent_off, the workgroup heads in d_wgs; d_apw with stripe pairs).
     bsp::SpmmStreamVariant stream_variant{};
@@ -186,6 +189,19 @@ void fill_info_sddmm(const bsp::SddmmSchedule& s, bsp_plan_info* info) {
     info->n_entries = (int32_t)s.ent_col.size();
     info->grid = (int32_t)s.wgmap.size();
     info->max_item_entries = s.max_item_entries;
+}
+
+void fill_info_sddmm_tiles(const bsp::SddmmTiles& s, bsp_plan_info* info) {
+    std::memset(info, 0, sizeof(*info));
+    const int32_t sub = (s.v.tile_m / bsp::kSub) * (s.cb / bsp::kSub);  // 32x32 sub-blocks of a chunk
+    info->kind = 2;
+    info->tile_n = s.v.tile_n;
+    info->n_items = s.n_items;
+    info->n_entries = (int32_t)s.ent_col.size() * sub;
+    info->grid = (int32_t)s.items.size();
+    info->max_item_entries = s.max_item_entries * sub;
+    info->stages = s.v.stages;
+    info->group = s.v.tile_m / bsp::kSub;
 }
 
 }  // namespace
@@ -759,8 +775,12 @@ int bsp_sddmm_plan_create(bsp_plan** out, const bsp_bsr_desc* mask, int64_t K, i
     int cus = 256;
     st = device_cus(device, &cus);
     if (st != BSP_OK) return st;
+    const bsp::SddmmTileVariant tv =
+        std::getenv("BSP_SDDMM_LOOP") ? bsp::SddmmTileVariant{} : bsp::sddmm_choose_tile(mask, K, cus);
+    const int tile_m = tv.tile_m;
     bsp::SddmmSchedule s;
-    st = bsp::build_sddmm_schedule(mask, K, cus, s, msg);
+    bsp::SddmmTiles ts;
+    st = tile_m ? bsp::build_sddmm_tiles(mask, K, cus, tv, ts, msg) : bsp::build_sddmm_schedule(mask, K, cus, s, msg);
     if (st != BSP_OK) return fail(st, msg);
 
     DeviceGuard g(device);
@@ -776,13 +796,20 @@ int bsp_sddmm_plan_create(bsp_plan** out, const bsp_bsr_desc* mask, int64_t K, i
     p->R = mask->R;
     p->C = mask->C;
     p->nblocks = mask->nblocks;
-    fill_info_sddmm(s, &p->info);
-    // BSP_SDDMM_LOOP selects the looped kernel for every K (for comparison).
-    p->sddmm_one_shot = bsp::sddmm_shot_supported(K, s.max_item_entries) && !std::getenv("BSP_SDDMM_LOOP");
-    p->info.stages = p->sddmm_one_shot ? 1 : 0;
-    hipError_t e = upload((bsp::SddmmItem**)&p->d_wgs, bsp::sddmm_wg_records(s));
-    if (e == hipSuccess) e = upload(&p->d_ent_row, s.ent_col);
-    if (e == hipSuccess) e = upload(&p->d_ent_off, s.ent_off);
+    if (tile_m) {
+        p->tile = tile_m;
+        p->sddmm_tile = tv;
+        for (int32_t w = ts.cb; w > 1; w >>= 1) ++p->cb_shift;
+        fill_info_sddmm_tiles(ts, &p->info);
+    } else {
+        fill_info_sddmm(s, &p->info);
+        // BSP_SDDMM_LOOP selects the looped kernel for every K (for comparison).
+        p->sddmm_one_shot = bsp::sddmm_shot_supported(K, s.max_item_entries) && !std::getenv("BSP_SDDMM_LOOP");
+        p->info.stages = p->sddmm_one_shot ? 1 : 0;
+    }
+    hipError_t e = upload((bsp::SddmmItem**)&p->d_wgs, tile_m ? ts.items : bsp::sddmm_wg_records(s));
+    if (e == hipSuccess) e = upload(&p->d_ent_row, tile_m ? ts.ent_col : s.ent_col);
+    if (e == hipSuccess) e = upload(&p->d_ent_off, tile_m ? ts.ent_off : s.ent_off);
     if (e == hipSuccess) e = hipDeviceSynchronize();
     if (e != hipSuccess) {
         free_plan_buffers(p);
@@ -810,6 +837,27 @@ int bsp_sddmm(const bsp_plan* p, const uint16_t* mask_vals, const uint16_t* x, i
         return fail(BSP_ERR_INVALID_ARGUMENT, "output or mask values misaligned");
     DeviceGuard g(p->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
+    if (p->tile) {
+        if (launch_skips() != 0)
+            return fail(BSP_ERR_UNSUPPORTED, "this plan's kernel has no switches to leave work out");
+        bsp::SddmmTileArgs ta{};
+        ta.mask = mask_vals;
+        ta.x = x;
+        ta.y = y;
+        ta.out = out_vals;
+        ta.items = (const bsp::SddmmItem*)p->d_wgs;
+        ta.ent_col = p->d_ent_row;
+        ta.ent_off = p->d_ent_off;
+        ta.ldx = ldx;
+        ta.ldy = ldy;
+        ta.ldo = (int32_t)p->C;
+        ta.K = (int32_t)p->K;
+        ta.cb_shift = p->cb_shift;
+        const hipError_t te = bsp::launch_sddmm_tile(ta, p->sddmm_tile, p->layout == BSP_COL_MAJOR,
+                                                     p->out_dtype == BSP_DTYPE_BF16, p->info.grid, (hipStream_t)stream);
+        if (te != hipSuccess) return hip_fail(te, "SDDMM launch");
+        return BSP_OK;
+    }
     bsp::SddmmArgs args{};
     args.mask = mask_vals;
     args.x = x;

@@ -18,6 +18,7 @@
 #include <cstdint>
 #include <cstdlib>
 
+#include "bsp_device.hpp"
 #include "bsp_kernels.hpp"
 #ifdef BSP_TIMELINE
 #include "bsparse_timeline.h"
@@ -86,60 +87,6 @@ struct TimelineGlobal {
 #define BSP_SKIP(p, bit) false
 #endif
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x4 __attribute__((ext_vector_type(4)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-
-typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-
-// fp32 -> bf16 with round-to-nearest-even: gfx950's v_cvt_pk_bf16_f32, which
-// converts two values per instruction.
-__device__ __forceinline__ uint16_t f32_to_bf16_rne(float f) {
-    return __builtin_bit_cast(uint16_t, (__bf16)f);
-}
-
-// Two values to packed bf16 (lo in bits 0-15).
-__device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
-    return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{lo, hi}, bf16x2));
-}
-
-__device__ __forceinline__ float bf16_to_f32(uint16_t h) {
-    return __uint_as_float((uint32_t)h << 16);
-}
-
-__device__ __forceinline__ f32x16 mfma32(const u32x4& a, const u32x4& b, const f32x16& c) {
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-// v_mfma_f32_16x16x32_bf16: lane l holds A[l%16][8*(l/16) .. +7] and
-// B[8*(l/16) .. +7][l%16]; result element v of lane l is D[4*(l/16) + v][l%16].
-__device__ __forceinline__ f32x4 mfma16(const u32x4& a, const u32x4& b, const f32x4& c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
-                                                   __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
-
-__device__ __forceinline__ uint32_t lds_address(const void* p) {
-    return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) uint8_t*)p;
-}
-
-// Reads plan data (written before the launch, never by a kernel) through the
-// constant address space so that it is fetched with scalar loads.
-template <typename T>
-__device__ __forceinline__ T load_const(const T* ptr) {
-    static_assert(sizeof(T) % 4 == 0, "plan records are whole dwords");
-    const __attribute__((address_space(4))) uint32_t* src =
-        (const __attribute__((address_space(4))) uint32_t*)(uintptr_t)ptr;
-    uint32_t w[sizeof(T) / 4];
-#pragma unroll
-    for (unsigned i = 0; i < sizeof(T) / 4; ++i) w[i] = src[i];
-    T out;
-    __builtin_memcpy(&out, w, sizeof(T));
-    return out;
-}
-
 // ---------------------------------------------------------------------------
 // SpMM.  Workgroup = one work item (a run of one 32-row stripe's sub-block
 // products) x one tile of TN = 128*NTW output columns; 4 waves, each owning
@@ -201,154 +148,7 @@ __device__ __forceinline__ int a_row_read_offset(int l32, int q, int s) {
     return 64 * l32 + 16 * ((2 * s + q) ^ ((l32 >> 2) & 3));
 }
 
-// Direct global->LDS load of 16 bytes per lane: lane L's bytes land at
-// lds_wave_base + 16*L (lds_wave_base is wave-uniform).  Issued as inline asm
-// so that the compiler does not track it: its own bookkeeping would otherwise
-// wait for every outstanding load before each LDS read or barrier, which
-// serialises the ring.  Completion is awaited explicitly with wait_vmcnt.
-// Nothing else in these kernels uses M0.
-__device__ __forceinline__ void gl_lds16(const void* g, uint32_t lds_wave_base) {
-    const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_wave_base);
-    __asm__ volatile(
-        "s_mov_b32 m0, %1\n\t"
-        "global_load_lds_dwordx4 %0, off"
-        :
-        : "v"(g), "s"(lds)
-        : "memory");
-}
-
-// The same load with a wave-uniform 64-bit base in SGPRs and a per-lane
-// 32-bit byte offset (the global saddr form): half the address data of the
-// 64-bit form, and the per-lane offset stays loop-invariant, so issuing a
-// product's loads needs no vector address arithmetic.
-__device__ __forceinline__ void gl_lds16_s(uint32_t voff_bytes, const void* sbase, uint32_t lds_wave_base) {
-    const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_wave_base);
-    __asm__ volatile(
-        "s_mov_b32 m0, %2\n\t"
-        "global_load_lds_dwordx4 %0, %1"
-        :
-        : "v"(voff_bytes), "s"(sbase), "s"(lds)
-        : "memory");
-}
-
-// The same with M0 = lds_base + IMM: one scalar add sets the LDS destination
-// (gl_lds16_s takes an add and a move).  The loader waves of the persistent
-// kernels issue several of these per entry, and a compute unit issues one
-// scalar instruction per cycle across all of its waves.
-template <int IMM>
-__device__ __forceinline__ void gl_lds16_si(uint32_t voff_bytes, const void* sbase, uint32_t lds_base) {
-    const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_base);
-    if constexpr (IMM == 0) {
-        __asm__ volatile(
-            "s_mov_b32 m0, %2\n\t"
-            "global_load_lds_dwordx4 %0, %1"
-            :
-            : "v"(voff_bytes), "s"(sbase), "s"(lds)
-            : "memory");
-    } else {
-        __asm__ volatile(
-            "s_add_u32 m0, %2, %3\n\t"
-            "global_load_lds_dwordx4 %0, %1"
-            :
-            : "v"(voff_bytes), "s"(sbase), "s"(lds), "n"(IMM)
-            : "memory", "scc");
-    }
-}
-
-// The same with 4 bytes per lane (lane i's dword lands at M0 + 4i).
-__device__ __forceinline__ void gl_lds4_s(uint32_t voff_bytes, const void* sbase, uint32_t lds_wave_base) {
-    const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_wave_base);
-    __asm__ volatile(
-        "s_mov_b32 m0, %2\n\t"
-        "global_load_lds_dword %0, %1"
-        :
-        : "v"(voff_bytes), "s"(sbase), "s"(lds)
-        : "memory");
-}
-
-// Workgroup barrier without a memory fence (a fence would wait for all
-// outstanding loads); the empty asm statements keep the compiler from moving
-// memory accesses across it.
-__device__ __forceinline__ void barrier_no_fence() {
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    __asm__ volatile("" ::: "memory");
-}
-
-// s_waitcnt with only the vector-memory counter constrained (gfx9 encoding:
-// vmcnt[3:0] bits 3:0, expcnt bits 6:4, lgkmcnt bits 11:8, vmcnt[5:4] bits 15:14).
-template <int N>
-__device__ __forceinline__ void wait_vmcnt() {
-    static_assert(N >= 0 && N < 64, "vmcnt out of range");
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt((N & 0xF) | (0x7 << 4) | (0xF << 8) | (((N >> 4) & 0x3) << 14));
-    __asm__ volatile("" ::: "memory");
-}
-
-// Waits until this wave's LDS accesses (and scalar loads) have completed.
-// The builtin, not inline asm: the compiler's own wait insertion then knows
-// that the LDS reads before it have returned, and adds no waits of its own
-// before later uses of the registers they wrote (with the asm form it kept
-// them pending and made the products of a step wait for the reads of the
-// next).
-__device__ __forceinline__ void wait_lgkm0() {
-    __asm__ volatile("" ::: "memory");
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    __asm__ volatile("" ::: "memory");
-}
-
-// Waits until at most PER*n + EXTRA vector loads of this wave are
-// outstanding, n <= NMAX.
-template <int PER, int NMAX, int EXTRA = 0>
-__device__ __forceinline__ void wait_stages(int n) {
-    if constexpr (NMAX >= 0) {
-        if (n >= NMAX) {
-            wait_vmcnt<PER * NMAX + EXTRA>();
-            return;
-        }
-        wait_stages<PER, NMAX - 1, EXTRA>(n);
-    }
-}
-
-// A pointer the compiler may hold in VGPRs made wave-uniform (SGPRs), for the
-// saddr operand of gl_lds16_s / gl_lds4_s, which must be an SGPR pair.  Only
-// for pointers that are uniform by construction (derived from plan words or
-// kernel arguments), where the compiler's divergence analysis loses that.
-template <typename T>
-__device__ __forceinline__ const T* uniform_ptr(const T* ptr) {
-    const uint64_t v = (uint64_t)(uintptr_t)ptr;
-    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
-    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
-    return (const T*)(uintptr_t)(((uint64_t)hi << 32) | lo);
-}
-
-__device__ __forceinline__ u32x4 ld_tr_b16(const uint8_t* lds) {
-    typedef short v4i16 __attribute__((ext_vector_type(4)));
-    v4i16 v = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-        (__attribute__((address_space(3))) v4i16*)(__attribute__((address_space(3))) uint8_t*)lds);
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    u32x2 w = __builtin_bit_cast(u32x2, v);
-    return u32x4{w.x, w.y, 0u, 0u};
-}
-
 }  // namespace spmm_detail
-
-// Output stores are non-temporal (global stores with nt: streamed through the
-// L2 without displacing the operands it holds, completing at the L2).  The
-// output is written once and never read by the kernel.  Against write-through
-// stores (sc1: a store that completes only when it has left the L2), measured
-// in one process on one MI355X, graph replay of the persistent SpMM kernel
-// with cold operands: 4096^2 x 512 fp32 C at 1% 5.50 -> 3.88 us, 5%
-// 6.29 -> 5.97 us, 25% 14.40 -> 14.10 us; the skewed 16384^2 x 1024 workload
-// 43.3 -> 39.7 us; the attention SDDMM 6.93 -> 6.55 us; the group kernels and
-// the fused attention kernel within 1%.  A wave that waits on vmcnt for loads
-// issued after its stores (the SpGEMM ring) would also wait for write-through
-// stores to leave the L2 (SpGEMM 8192^2 fp32: 108 us with them, 28 us with
-// non-temporal stores).
-template <typename T>
-__device__ __forceinline__ void store_out(T* p, T v) {
-    __builtin_nontemporal_store(v, p);
-}
 
 // Stores one 32x32 MFMA result at rows row0.., column col (this lane's
 // column; skipped past N).

@@ -183,6 +183,26 @@ inline bool sddmm_shot_supported(int64_t K, int max_item_entries) {
     return (K == 32 || K == 64 || K == 128 || K == 256) && max_item_entries <= 4;
 }
 
+// SDDMM on tiles of tile_m rows x up to tile_n gathered columns
+// (sddmm_tile_kernel, any K).
+struct SddmmTileArgs {
+    const uint16_t* mask;     // mask block values (bf16), nblocks*R*C
+    const uint16_t* x;        // X (bf16), row-major M x K, leading dim ldx
+    const uint16_t* y;        // Y (bf16), K x N row-major or N x K row-major (col-major Y)
+    void* out;                // output block values (fp32 or bf16), nblocks*R*C
+    const SddmmItem* items;   // one record per workgroup (empty range: idle)
+    const int32_t* ent_col;   // first column of Y per column chunk
+    const int64_t* ent_off;   // element offset of the chunk's first output value (row x_row0)
+    int64_t ldx;
+    int64_t ldy;
+    int32_t ldo;              // row stride inside an output / mask block (= C)
+    int32_t K;
+    int32_t cb_shift;         // log2 of the chunk width in columns
+    int32_t pad;
+};
+hipError_t launch_sddmm_tile(const SddmmTileArgs& a, const SddmmTileVariant& v, bool y_colmajor, bool out_bf16, int grid,
+                             hipStream_t stream);
+
 struct SpgemmArgs {
     const uint16_t* a;          // A block values (bf16), R x C blocks
     const uint16_t* b;          // B block values (bf16), C x BC blocks

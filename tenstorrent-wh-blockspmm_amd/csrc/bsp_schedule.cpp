@@ -13,6 +13,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <cstdio>
 #include <cstdlib>
 #include <numeric>
 #include <queue>
@@ -1438,6 +1439,201 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
     s.runs.assign((size_t)s.grid * 4, SpgemmRun{(int32_t)ntask, (int32_t)ntask, pend, pend});
     for (int x = 0; x < kNumXcd; ++x)
         std::copy(region_runs[x].begin(), region_runs[x].end(), s.runs.begin() + (size_t)x * per * 4);
+    return BSP_OK;
+}
+
+// When the tile kernel takes an SDDMM, E being the mask's 32x32 sub-blocks
+// (4096^2, fp32 out, row-major Y, us of the 32-row kernels : best tile):
+//   - K > 256 (past the one-shot kernel) and E >= 2 per compute unit.  Fewer
+//     leave most tiles' compute units idle, where the looped kernel splits K
+//     over its waves (1024^2 10%, K = 320: 3.7 : 4.7; 4096^2 5%, K = 320, 32 /
+//     64 / 256-row blocks: 8.5 : 7.5, 8.1 : 6.6, 7.2 : 5.4; 25%, K = 512:
+//     34.2 : 19.5, 34.6 : 14.4, 38.4 : 12.6);
+//   - K of 96 to 256, blocks of 64 rows or more and E > 8 per compute unit
+//     (more than one round of one-shot items): 25%, K = 96 / 256: 9.0 : 7.5,
+//     12.2 : 10.0 (64-row blocks), 9.6 : 7.3, 12.3 : 9.2 (256); at 5% (E = 3
+//     per compute unit) 3.8 : 4.2 and 4.7 : 5.5, at K = 64 6.3 : 7.1;
+//   - K of 192 to 256, blocks of 32 rows and E >= 32 per compute unit (8192^2
+//     25%, K = 256: 37.0 : 32.7; K = 128 22.5 : 23.7).
+// Which tile: an estimate of its time, us = steps x max(latency, m x rate) +
+// m x (its epilogue), m the items a compute unit gets (past one round of
+// resident workgroups, 0.4 of a round more: the last one is partly empty) and
+// steps = K / 64.  The
+// constants are fitted to 4096^2 and 8192^2 masks of 5% and 25%, K = 256 to
+// 8192, blocks of 32 to 256 (the estimate's pick was within 8% of the best
+// tile on all of them).  With few items per compute unit, deeper rings: 4096^2
+// 5% K = 2048 32 x 128 tiles 20.3 -> 16.8 us, 64 x 128 21.8 -> 18.7.
+SddmmTileVariant sddmm_choose_tile(const bsp_bsr_desc* m, int64_t K, int num_cus) {
+    if (num_cus <= 0) num_cus = 256;
+    SddmmTileVariant v{};
+    if (const char* e = std::getenv("BSP_SDDMM_TILE")) {  // "rows,columns,stages" of a compiled tile; else none
+        SddmmTileVariant f{};
+        if (std::sscanf(e, "%d,%d,%d", &f.tile_m, &f.tile_n, &f.stages) == 3 && f.tile_m > 0 && m->R % f.tile_m == 0) {
+#define BSP_SDDMM_TILE_MATCH(TM, TN, WR, WC, S, CH, WPE) \
+    if (f.tile_m == TM && f.tile_n == TN && f.stages == S) return f;
+            BSP_SDDMM_TILES(BSP_SDDMM_TILE_MATCH)
+#undef BSP_SDDMM_TILE_MATCH
+        }
+        return v;
+    }
+    if (m->R <= 0 || m->C <= 0 || m->R % kSub || m->C % kSub) return v;
+    const int64_t E = m->nblocks * (m->R / kSub) * (m->C / kSub);
+    const bool rows64 = m->R % 64 == 0;
+    if (!(K > 256 ? E >= 2 * (int64_t)num_cus
+                  : rows64 ? K >= 96 && E > 8 * (int64_t)num_cus : K >= 192 && E >= 32 * (int64_t)num_cus))
+        return v;
+    struct Cost {
+        int tm, tn;
+        double lat, rate, epilogue;
+    };
+    static const Cost costs[] = {{32, 128, 0.62, 0.27, 1.1},
+                                 {64, 128, 0.66, 0.43, 1.9},
+                                 {128, 128, 0.88, 0.73, 3.5},
+                                 {256, 256, 2.0, 2.1, 18.0}};
+    const double steps = (double)((K + 63) / 64);
+    double best = 0;
+    int64_t best_items = 0;
+    for (const Cost& c : costs) {
+        if (m->R % c.tm) continue;
+        int64_t cb = kSub;
+        while (cb * 2 <= c.tn && m->C % (cb * 2) == 0) cb *= 2;
+        const int64_t per = m->C / cb, G = c.tn / cb;
+        int64_t items = 0;
+        for (int64_t r = 0; r < m->H / m->R; ++r) items += ((m->indptr[r + 1] - m->indptr[r]) * per + G - 1) / G;
+        items *= m->R / c.tm;
+        const int wgs = sddmm_tile_wgs({c.tm, c.tn, 2});
+        const double each = std::max(1.0, (double)items / num_cus) + (items > (int64_t)num_cus * wgs ? 0.4 * wgs : 0.0);
+        const double t = steps * std::max(c.lat, each * c.rate) + each * c.epilogue;
+        if (!v.tile_m || t < best) best = t, v.tile_m = c.tm, v.tile_n = c.tn, best_items = items;
+    }
+    v.stages = 2;
+    if (steps >= 8 && v.tile_m == 32 && best_items <= num_cus) v.stages = 4;
+    if (steps >= 8 && v.tile_m == 64 && best_items <= num_cus) v.stages = 3;
+    return v;
+}
+
+int build_sddmm_tiles(const bsp_bsr_desc* m, int64_t K, int num_cus, const SddmmTileVariant& v, SddmmTiles& s,
+                      std::string& msg) {
+    const int tile_m = v.tile_m;
+    int st = validate_bsr(m, msg);
+    if (st != BSP_OK) return st;
+    if (K <= 0) {
+        msg = "K must be positive";
+        return BSP_ERR_INVALID_ARGUMENT;
+    }
+    if (m->R % kSub || m->C % kSub || K % kSub || tile_m < kSub || m->R % tile_m) {
+        msg = "R, C and K must be multiples of 32";
+        return BSP_ERR_UNSUPPORTED;
+    }
+    if (num_cus <= 0) num_cus = 256;
+    s = SddmmTiles{};
+    s.v = v;
+    s.cb = kSub;
+    while (s.cb * 2 <= v.tile_n && m->C % (s.cb * 2) == 0) s.cb *= 2;
+    const int64_t G = v.tile_n / s.cb;       // chunks per item
+    const int64_t CS = m->C / s.cb;          // chunks per block
+    const int64_t RS = m->R / tile_m;        // stripes per block row
+    const int64_t nbr = m->H / m->R, nbc = m->W / m->C;
+    if (m->nblocks * (m->R / kSub) * (m->C / kSub) > INT32_MAX || m->W > INT32_MAX || m->H > INT32_MAX || K > INT32_MAX) {
+        msg = "problem too large for int32 schedule fields";
+        return BSP_ERR_UNSUPPORTED;
+    }
+    const int64_t slots = (int64_t)num_cus * sddmm_tile_wgs(v);
+
+    // Column groups cg in {1, 2, 4, 8} of block columns crossed with 8 / cg row
+    // groups of block rows, both of about equal block counts; region x = row
+    // group * cg + column group goes to XCD x.  Taken: the fewest rounds of
+    // resident workgroups, then the fewest bytes the XCDs read in all (each
+    // region's distinct stripes of X and column blocks of Y).
+    std::vector<int64_t> colcnt(nbc, 0);
+    for (int64_t e = 0; e < m->nblocks; ++e) ++colcnt[m->indices[e]];
+    std::vector<int32_t> best_cg_of, best_rg_of;
+    int best_cg = 0;
+    int64_t best_rounds = 0, best_bytes = 0;
+    for (int cg = 1; cg <= kNumXcd; cg *= 2) {
+        const int rg = kNumXcd / cg;
+        if (cg > 1 && cg > nbc) break;
+        std::vector<int32_t> cg_of(nbc), rg_of(nbr);
+        int64_t run = 0;
+        for (int64_t c = 0; c < nbc; ++c) {
+            cg_of[c] = (int32_t)std::min<int64_t>(cg - 1, m->nblocks ? run * cg / m->nblocks : 0);
+            run += colcnt[c];
+        }
+        for (int64_t r = 0; r < nbr; ++r)
+            rg_of[r] = (int32_t)std::min<int64_t>(rg - 1, m->nblocks ? (int64_t)m->indptr[r] * rg / m->nblocks : 0);
+        int64_t items = 0, bytes = 0;
+        std::vector<int64_t> cnt(cg);
+        std::vector<uint8_t> seen((size_t)kNumXcd * nbc, 0);
+        for (int64_t r = 0; r < nbr; ++r) {
+            std::fill(cnt.begin(), cnt.end(), 0);
+            for (int32_t e = m->indptr[r]; e < m->indptr[r + 1]; ++e) {
+                const int g = cg_of[m->indices[e]];
+                ++cnt[g];
+                uint8_t& f = seen[(size_t)(rg_of[r] * cg + g) * nbc + m->indices[e]];
+                if (!f) bytes += m->C;
+                f = 1;
+            }
+            for (int g = 0; g < cg; ++g) {
+                items += RS * ((cnt[g] * CS + G - 1) / G);
+                if (cnt[g]) bytes += m->R;
+            }
+        }
+        const int64_t rounds = (items + slots - 1) / slots;
+        if (!best_cg || rounds < best_rounds || (rounds == best_rounds && bytes < best_bytes)) {
+            best_cg = cg, best_rounds = rounds, best_bytes = bytes;
+            best_cg_of.swap(cg_of);
+            best_rg_of.swap(rg_of);
+        }
+    }
+
+    // Items: each stripe's chunks of one column group in equal runs of at most G.
+    std::vector<SddmmItem> items;
+    std::vector<std::vector<int32_t>> bins(kNumXcd);
+    std::vector<std::vector<int32_t>> groups(best_cg);
+    for (int64_t r = 0; r < nbr; ++r) {
+        for (auto& g : groups) g.clear();
+        for (int32_t e = m->indptr[r]; e < m->indptr[r + 1]; ++e) groups[best_cg_of[m->indices[e]]].push_back(e);
+        for (int g = 0; g < best_cg; ++g) {
+            const int64_t n = (int64_t)groups[g].size() * CS;
+            if (!n) continue;
+            const int64_t pieces = (n + G - 1) / G;
+            for (int64_t sub = 0; sub < RS; ++sub) {
+                const int64_t e0 = (int64_t)s.ent_col.size();
+                for (int32_t e : groups[g])
+                    for (int64_t t = 0; t < CS; ++t) {
+                        s.ent_col.push_back((int32_t)((int64_t)m->indices[e] * m->C + t * s.cb));
+                        s.ent_off.push_back((int64_t)e * m->R * m->C + sub * tile_m * m->C + t * s.cb);
+                    }
+                for (int64_t q = 0; q < pieces; ++q) {
+                    const int64_t b = e0 + q * n / pieces, d = e0 + (q + 1) * n / pieces;
+                    bins[best_rg_of[r] * best_cg + g].push_back((int32_t)items.size());
+                    items.push_back({(int32_t)(r * m->R + sub * tile_m), (int32_t)b, (int32_t)d, 0});
+                    s.max_item_entries = std::max<int32_t>(s.max_item_entries, (int32_t)(d - b));
+                }
+            }
+        }
+    }
+    s.n_items = (int32_t)items.size();
+    // Equal counts: what a region has over its share goes to the XCDs with room.
+    const size_t cap = (items.size() + kNumXcd - 1) / kNumXcd;
+    std::vector<int32_t> spare;
+    for (auto& b : bins)
+        while (b.size() > cap) {
+            spare.push_back(b.back());
+            b.pop_back();
+        }
+    for (auto& b : bins) {
+        while (b.size() < cap && !spare.empty()) {
+            b.push_back(spare.back());
+            spare.pop_back();
+        }
+        std::stable_sort(b.begin(), b.end(), [&](int32_t x, int32_t y) {
+            return items[x].e_end - items[x].e_begin > items[y].e_end - items[y].e_begin;
+        });
+    }
+    s.items.assign(cap * kNumXcd, SddmmItem{0, 0, 0, 0});
+    for (int x = 0; x < kNumXcd; ++x)
+        for (size_t j = 0; j < bins[x].size(); ++j) s.items[j * kNumXcd + x] = items[bins[x][j]];
     return BSP_OK;
 }
 

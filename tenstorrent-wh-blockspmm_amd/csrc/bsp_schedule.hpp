@@ -2,6 +2,7 @@
 // walk.  Pure C++ (no HIP), so it runs and is tested without a device.
 #pragma once
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -296,6 +297,45 @@ struct SddmmSchedule {
 
 // Per-workgroup items in launch order; idle slots get an empty range.
 std::vector<SddmmItem> sddmm_wg_records(const SddmmSchedule& s);
+
+// ---- SDDMM tiles (sddmm_tile_kernel) ----------------------------------------
+// An item is tile_m rows of one block row times up to tile_n / cb column
+// chunks of cb columns gathered from its stored blocks; a workgroup each.
+//
+// Compiled tiles: rows, columns, wave grid (rows x columns), ring stages,
+// accumulation chains, waves per SIMD.  LDS = 128 (rows + columns) x stages.
+#define BSP_SDDMM_TILES(X)      \
+    X(32, 128, 1, 4, 2, 4, 4)   \
+    X(32, 128, 1, 4, 4, 4, 2)   \
+    X(64, 128, 2, 2, 2, 2, 3)   \
+    X(64, 128, 2, 2, 3, 2, 2)   \
+    X(128, 128, 2, 2, 2, 2, 2)  \
+    X(256, 256, 2, 4, 2, 1, 2)
+struct SddmmTileVariant {
+    int tile_m = 0;  // 0: no tile kernel
+    int tile_n = 0;
+    int stages = 0;
+};
+// Workgroups of a variant that a compute unit holds (LDS).
+inline int sddmm_tile_wgs(const SddmmTileVariant& v) {
+    return std::max(1, 160 * 1024 / (128 * (v.tile_m + v.tile_n) * v.stages));
+}
+struct SddmmTiles {
+    SddmmTileVariant v;
+    int32_t cb = 0;                // chunk width: the largest of 256, 128, 64, 32 that divides C and tile_n
+    int32_t max_item_entries = 0;  // chunks
+    int32_t n_items = 0;
+    std::vector<SddmmItem> items;  // in launch order (workgroup g on XCD g % kNumXcd); idle slots empty
+    std::vector<int32_t> ent_col;  // first column of Y of the chunk
+    std::vector<int64_t> ent_off;  // element offset of its first output value (row x_row0)
+};
+// The tile a plan takes (tile_m 0: none, the 32-row kernels run): see the
+// definition for the rule.
+SddmmTileVariant sddmm_choose_tile(const bsp_bsr_desc* mask, int64_t K, int num_cus);
+// Items of v.tile_m rows (dividing R), spread over the XCDs in a 2-D split of
+// block rows and columns.
+int build_sddmm_tiles(const bsp_bsr_desc* mask, int64_t K, int num_cus, const SddmmTileVariant& v, SddmmTiles& s,
+                      std::string& msg);
 
 // One SpGEMM wave task: a 32x32 output sub-block and its run of products.
 struct SpgemmTask {

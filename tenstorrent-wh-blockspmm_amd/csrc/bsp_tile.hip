@@ -1,0 +1,430 @@
+// Tile kernel: SDDMM with long K or large blocks, each workgroup computing a
+// TM x TN output tile (gfx950).
+//
+// A tile is a product of an A panel, TM rows contiguous along k (X rows, rows
+// of an A block), and a B panel of TN columns, along k in steps of 64.  A step
+// is one stage of an S-stage LDS ring filled by direct global->LDS loads:
+//   - rows contiguous along k ("k-rows": A, and B when it is stored
+//     transposed) take 128 bytes per step, row r at 128 r, its 16-byte chunk c
+//     at slot c ^ ((r >> 1) & 7).  A load instruction fetches eight rows, 128
+//     contiguous bytes (one cache line) each.  A 16-lane quarter of an operand
+//     read takes one chunk of 16 consecutive rows, which the XOR spreads over
+//     all 64 banks;
+//   - rows contiguous along the columns ("n-rows": row-major B) take 2 TN
+//     bytes, 64 of them per step, row k's chunk c at slot c ^ 4 (k % 4) (at 64
+//     columns, where a row is half the banks, c ^ 4 (k / 2 % 2)), read back by
+//     transpose reads (as in the SpMM kernels).
+// A wave holds FM x FN MFMA tiles of 32 x 32 and reads each 16-deep k-step's
+// operands into one of two register sets while it multiplies the other's.  The
+// last k-step's products of a stage are issued behind the barrier that
+// publishes the next stage, beside its first reads: one barrier per 64-deep
+// step, and no part of a step is reads alone.
+//
+// Reference semantics: sparse_common/bsr_matrix.hpp:816-857.
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "bsp_device.hpp"
+#include "bsp_kernels.hpp"
+
+namespace bsp {
+
+namespace tile_detail {
+
+using namespace spmm_detail;
+
+// One workgroup's share of the tile product: operand layout, reads, products
+// and the ring.  BK: B is stored k-rows (transposed); else n-rows.
+template <int TM, int TN, int WR, int WC, int S, bool BK, int CH = 1>
+struct Tile {
+    static constexpr int NW = WR * WC;             // waves
+    static constexpr int FM = TM / 32 / WR;        // 32-row MFMA tiles per wave
+    static constexpr int FN = TN / 32 / WC;        // 32-column MFMA tiles per wave
+    static constexpr int A_BYTES = TM * 128;       // per stage
+    static constexpr int B_BYTES = TN * 128;
+    static constexpr int STAGE = A_BYTES + B_BYTES;
+    static constexpr int AL = TM / 8 / NW;         // 1 KB loads per wave and stage
+    static constexpr int BL = TN / 8 / NW;
+    static constexpr int PER = AL + BL;
+    static constexpr int LDS = S * STAGE;
+    static_assert(AL * NW * 8 == TM && BL * NW * 8 == TN, "whole loads per wave");
+    static_assert(PER * S < 64, "vmcnt budget");
+
+    int lane, wave, l32, q, wr, wc;
+    uint32_t lds0;
+    const uint8_t* smem;
+    int a_rd[4];                  // A: byte offset of k-step s (+ 4096 per 32 rows)
+    int b_rd[BK ? 4 : FN];        // B: as A, or per 32-column tile (+ 32 TN per k-step, 8 TN per row group)
+    f32x16 acc[FM][FN];
+    f32x16 part[CH > 1 ? CH - 1 : 1][FM][FN];  // the other chains' sums
+
+    // What the slot of n-row r's chunk differs by.
+    static __device__ __forceinline__ int nswz(int r) { return TN >= 128 ? 4 * (r & 3) : 4 * ((r >> 1) & 1); }
+
+    struct Ops {
+        u32x4 a[FM];
+        u32x4 b[FN];
+    };
+
+    __device__ __forceinline__ explicit Tile(const uint8_t* lds) {
+        lane = threadIdx.x & 63;
+        wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+        l32 = lane & 31;
+        q = lane >> 5;
+        wr = wave / WC;
+        wc = wave % WC;
+        smem = lds;
+        lds0 = lds_address(lds);
+        const int row = l32 * 128, x = (l32 >> 1) & 7;
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            a_rd[s] = wr * FM * 4096 + row + 16 * ((2 * s + q) ^ x);
+            if constexpr (BK) b_rd[s] = A_BYTES + wc * FN * 4096 + row + 16 * ((2 * s + q) ^ x);
+        }
+        if constexpr (!BK) {
+#pragma unroll
+            for (int nt = 0; nt < FN; ++nt) {
+                const int g = lane >> 4;
+                const int r = 8 * (g >> 1) + ((lane & 15) >> 2);
+                const int col = (wc * FN + nt) * 32 + 16 * (g & 1) + 4 * (lane & 3);
+                b_rd[nt] = A_BYTES + r * (2 * TN) + 16 * ((col >> 3) ^ nswz(r)) + 2 * (col & 7);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int nt = 0; nt < FN; ++nt)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    acc[i][nt][v] = 0.0f;
+#pragma unroll
+                    for (int c = 0; c + 1 < CH; ++c) part[c][i][nt][v] = 0.0f;
+                }
+    }
+
+    // What lane `lane` of this wave's load j fetches.  k-rows: row of the
+    // panel and chunk of its 128 bytes; n-rows: k of the step and chunk.
+    __device__ __forceinline__ int krow(int j, int per) const { return 8 * (wave * per + j) + (lane >> 3); }
+    __device__ __forceinline__ int kchunk(int j, int per) const {
+        return (lane & 7) ^ ((krow(j, per) >> 1) & 7);
+    }
+    __device__ __forceinline__ int nrow(int j) const {
+        return ((wave * BL + j) * 1024 + lane * 16) / (2 * TN);
+    }
+    __device__ __forceinline__ int nchunk(int j) const {
+        return (((wave * BL + j) * 1024 + lane * 16) % (2 * TN)) / 16 ^ nswz(nrow(j));
+    }
+    __device__ __forceinline__ uint32_t a_lds(int stage, int j) const {
+        return lds0 + stage * STAGE + (wave * AL + j) * 1024;
+    }
+    __device__ __forceinline__ uint32_t b_lds(int stage, int j) const {
+        return lds0 + stage * STAGE + A_BYTES + (wave * BL + j) * 1024;
+    }
+
+    __device__ __forceinline__ void read(int stage, int s, Ops& o) const {
+        const uint8_t* st = smem + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < FM; ++i) o.a[i] = *(const u32x4*)(st + a_rd[s] + i * 4096);
+#pragma unroll
+        for (int nt = 0; nt < FN; ++nt) {
+            if constexpr (BK) {
+                o.b[nt] = *(const u32x4*)(st + b_rd[s] + nt * 4096);
+            } else {
+                const u32x4 lo = ld_tr_b16(st + b_rd[nt] + s * 32 * TN);
+                const u32x4 hi = ld_tr_b16(st + b_rd[nt] + s * 32 * TN + 8 * TN);
+                o.b[nt] = u32x4{lo.x, lo.y, hi.x, hi.y};
+            }
+        }
+    }
+    // Products of k-step s of a stage, into chain s % CH.
+    __device__ __forceinline__ void mul(const Ops& o, int s) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int nt = 0; nt < FN; ++nt) {
+                f32x16& c = s % CH == 0 ? acc[i][nt] : part[CH > 1 ? s % CH - 1 : 0][i][nt];
+                c = mfma32(o.a[i], o.b[nt], c);
+            }
+    }
+    // Adds the chains, once the last products have left the matrix core: a
+    // VALU read of an MFMA result needs wait states after it (11 here), which
+    // the compiler (ROCm 7.2) does not insert where a branch leads from the
+    // products to the sum (the half step's end: the sums of its second k-step
+    // were lost), so the wait is written here and the sums tied behind it.
+    __device__ __forceinline__ void fold() {
+        __asm__ volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int nt = 0; nt < FN; ++nt) {
+                __asm__ volatile("" : "+v"(acc[i][nt]));
+#pragma unroll
+                for (int c = 0; c + 1 < CH; ++c) __asm__ volatile("" : "+v"(part[c][i][nt]));
+            }
+#pragma unroll
+        for (int c = 0; c + 1 < CH; ++c)
+#pragma unroll
+            for (int i = 0; i < FM; ++i)
+#pragma unroll
+                for (int nt = 0; nt < FN; ++nt) acc[i][nt] += part[c][i][nt];
+    }
+    // The reads of the next k-step go between the first half of the products.
+    __device__ __forceinline__ void interleave() const {
+        constexpr int MF = FM * FN, RD = FM + (BK ? FN : 2 * FN);
+        constexpr int SPAN = MF > 1 ? MF / 2 : 1, PERM = (RD + SPAN - 1) / SPAN;
+#pragma unroll
+        for (int i = 0; i < SPAN; ++i) {
+            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);     // one MFMA
+            __builtin_amdgcn_sched_group_barrier(0x100, PERM, 0);  // LDS reads
+        }
+        if constexpr (MF > SPAN) __builtin_amdgcn_sched_group_barrier(0x008, MF - SPAN, 0);
+    }
+
+    // n steps of 64 (the last one 32 deep with `half_tail`); issue(k, stage)
+    // issues this wave's PER loads of step k, steps in ascending order.  A wave that is not `live`
+    // (no output) loads and meets the barriers only.  Ends with every wave's
+    // reads complete (the ring may be overwritten after a barrier).
+    template <class Issue>
+    __device__ __forceinline__ void run(int n, bool half_tail, bool live, Issue&& issue) {
+#pragma unroll
+        for (int k = 0; k < S; ++k)
+            if (k < n) issue(k, k);
+        wait_stages<PER, S - 1>(min(S, n) - 1);  // step 0 landed
+        barrier_no_fence();
+        auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
+        Ops o0, o1;
+        if (live) read(0, 0, o0);
+        fence();
+        int stage = 0;
+        for (int k = 0; k + 1 < n; ++k) {
+            if (live) {
+                mul(o0, 0);
+                read(stage, 1, o1);
+                interleave();
+                fence();
+                mul(o1, 1);
+                read(stage, 2, o0);
+                interleave();
+                fence();
+                mul(o0, 2);
+                read(stage, 3, o1);
+                interleave();
+                fence();
+            }
+            wait_lgkm0();
+            if (k + S < n)
+                wait_vmcnt<PER * (S - 2)>();  // step k+1 landed; k+2 .. k+S-1 in flight
+            else
+                wait_stages<PER, S - 2>(n - 2 - k);
+            barrier_no_fence();
+            if (k + S < n) issue(k + S, stage);
+            stage = stage == S - 1 ? 0 : stage + 1;
+            if (live) {
+                mul(o1, 3);
+                read(stage, 0, o0);
+                interleave();
+            }
+            fence();
+        }
+        if (live) {
+            mul(o0, 0);
+            read(stage, 1, o1);
+            interleave();
+            fence();
+            mul(o1, 1);
+            if (!half_tail) {
+                read(stage, 2, o0);
+                fence();
+                mul(o0, 2);
+                read(stage, 3, o1);
+                interleave();
+                fence();
+                mul(o1, 3);
+            }
+            fold();
+        }
+        wait_lgkm0();
+    }
+};
+
+}  // namespace tile_detail
+
+// ---------------------------------------------------------------------------
+// SDDMM.  A workgroup takes TM rows of one block row and up to TN columns
+// gathered from its stored blocks: `cb`-wide column chunks (cb divides C and
+// TN), each with its column of Y and its place in the output.  X's rows then
+// serve TN columns and each column of Y serves TM rows, where the one-shot
+// and looped kernels load Y anew for every 32 rows.
+//
+// What bounds it: the largest tile, on full 256 x 256 blocks and long K, the
+// matrix cores at the clock they hold (8192^3, 25%: 2730 -> 255-270 us, 1.02-
+// 1.08 PFLOP/s); the small ones the latency of a step's loads, which several
+// workgroups of a compute unit hide in turn (4096^2, 32 x 32 blocks, 25%,
+// K = 512: 34-41 -> 17-19 us; two stages and four workgroups beat four stages
+// and two, 19.6 : 22.3).  The 128 and 64-row tiles are for masks whose blocks
+// or counts do not fill the compute units with larger ones (see
+// sddmm_choose_tile).  CH chains of partial sums, taken in turn by the k-steps
+// of a stage, keep the error of a long sum down where registers allow (fp32
+// out, K = 2048, against 64 bits: four chains 1.3e-7, one 2.7e-7, and the
+// looped kernel, whose waves split K in four, 1.3e-7).
+template <int TM, int TN, int WR, int WC, int S, bool YT, bool OUT_BF16, int CH, int WPE>
+__global__ __launch_bounds__(64 * WR * WC, WPE) void sddmm_tile_kernel(SddmmTileArgs p) {
+    using namespace tile_detail;
+    using T = Tile<TM, TN, WR, WC, S, YT, CH>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[T::LDS];
+    const SddmmItem it = load_const(p.items + blockIdx.x);
+    const int nc = it.e_end - it.e_begin;  // column chunks
+    if (nc <= 0) return;                   // idle slot (uniform)
+    T t(smem);
+    const int lane = t.lane;
+    const int cbs = p.cb_shift;  // log2(cb)
+    auto chunk_of = [&](int col) { return min(col >> cbs, nc - 1); };  // past the last chunk: that chunk again
+
+    // Per-lane source of loads 0 and 1 of each panel, advanced by one step per
+    // issue.  Loads two apart differ by a whole number of rows (16 k-rows, four
+    // n-rows) and take the same chunk; a wave's 32 k-rows of Y lie in one chunk.
+    constexpr int NPX = T::AL < 2 ? 1 : 2, NPY = T::BL < 2 ? 1 : 2;
+    static_assert(8 * T::BL <= 32, "a wave's rows of Y^T lie in one column chunk");
+    const uint8_t *px[NPX], *py[NPY];
+#pragma unroll
+    for (int j = 0; j < NPX; ++j)
+        px[j] = (const uint8_t*)(p.x + (int64_t)(it.x_row0 + t.krow(j, T::AL)) * p.ldx + 8 * t.kchunk(j, T::AL));
+#pragma unroll
+    for (int j = 0; j < NPY; ++j) {
+        if constexpr (YT) {
+            const int r = t.krow(j, T::BL);
+            const int64_t col = p.ent_col[it.e_begin + chunk_of(r)] + (r & ((1 << cbs) - 1));
+            py[j] = (const uint8_t*)(p.y + col * p.ldy + 8 * t.kchunk(j, T::BL));
+        } else {
+            const int c = 8 * t.nchunk(j);
+            const int64_t col = p.ent_col[it.e_begin + chunk_of(c)] + (c & ((1 << cbs) - 1));
+            py[j] = (const uint8_t*)(p.y + (int64_t)t.nrow(j) * p.ldy + col);
+        }
+    }
+    const int n = (p.K + 63) >> 6;
+    const bool half_tail = (p.K & 63) != 0;
+    const int64_t ystep = YT ? 128 : 128 * p.ldy;
+    const int64_t xtwo = 32 * p.ldx, ytwo = (YT ? 32 : 2048 / TN) * p.ldy;  // bytes between loads j and j + 2
+    auto issue = [&](int k, int stage) {
+        if (half_tail && k == n - 1) {
+            // The second half of the last step is past K: fetch its first
+            // half twice (those products are not made).
+#pragma unroll
+            for (int j = 0; j < NPX; ++j)
+                if (t.kchunk(j, T::AL) >= 4) px[j] -= 64;
+#pragma unroll
+            for (int j = 0; j < NPY; ++j)
+                if (YT && t.kchunk(j, T::BL) >= 4) py[j] -= 64;
+        }
+#pragma unroll
+        for (int j = 0; j < T::AL; ++j) gl_lds16(px[j % 2] + (j / 2) * xtwo, t.a_lds(stage, j));
+#pragma unroll
+        for (int j = 0; j < T::BL; ++j) {
+            const uint8_t* src = py[j % 2] + (j / 2) * ytwo;
+            if (!YT && half_tail && k == n - 1 && t.nrow(j) >= 32) src -= 64 * p.ldy;
+            gl_lds16(src, t.b_lds(stage, j));
+        }
+#pragma unroll
+        for (int j = 0; j < NPX; ++j) px[j] += 128;
+#pragma unroll
+        for (int j = 0; j < NPY; ++j) py[j] += ystep;
+    };
+    const bool live = ((t.wc * T::FN * 32) >> cbs) < nc;
+    t.run(n, half_tail, live, issue);
+
+    // The mask tile comes through the ring's LDS as n-rows of TN values (16-byte
+    // loads; transpose reads give the accumulators' layout), or value by value
+    // if the mask is not 16-byte aligned.
+    constexpr int ML = TM * TN * 2 / 1024 / T::NW;  // 1 KB loads per wave
+    static_assert(TM * TN * 2 <= T::LDS && ML % 2 == 0, "mask tile fits the ring");
+    const bool mask16 = ((uintptr_t)p.mask & 15u) == 0;
+    barrier_no_fence();
+    if (mask16) {
+        constexpr int RPL = 512 / TN;  // rows per load (2 at 256 columns, 4 at 128)
+        static_assert(RPL == 2 || RPL == 4, "rows per load");
+        int64_t src[4 / RPL];
+#pragma unroll
+        for (int h = 0; h < 4 / RPL; ++h) {
+            const int row = h * RPL + lane / (TN / 8);
+            const int c = 8 * ((lane % (TN / 8)) ^ (4 * (row & 3)));
+            src[h] = p.ent_off[it.e_begin + chunk_of(c)] + (int64_t)row * p.ldo + (c & ((1 << cbs) - 1));
+        }
+#pragma unroll
+        for (int j = 0; j < ML; ++j) {
+            const int I = t.wave * ML + j;  // rows RPL * I ..
+            gl_lds16(p.mask + src[RPL == 2 ? j & 1 : 0] + (int64_t)(RPL * I & ~3) * p.ldo, t.lds0 + I * 1024);
+        }
+        wait_vmcnt<0>();
+    }
+    barrier_no_fence();
+    if (!live) return;
+#pragma unroll
+    for (int nt = 0; nt < T::FN; ++nt) {
+        const int c0 = (t.wc * T::FN + nt) * 32;
+        const int g = c0 >> cbs;
+        if (g >= nc) break;
+        const int64_t off = load_const(p.ent_off + it.e_begin + g) + (c0 & ((1 << cbs) - 1)) + t.l32;
+#pragma unroll
+        for (int i = 0; i < T::FM; ++i) {
+            const int row0 = (t.wr * T::FM + i) * 32 + 4 * t.q;
+            uint32_t mk[16];
+            if (mask16) {
+#pragma unroll
+                for (int v4 = 0; v4 < 4; ++v4) {
+                    const int row = row0 + 8 * v4 + ((lane & 15) >> 2);
+                    const int col = c0 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+                    const u32x4 r = ld_tr_b16(smem + row * (2 * TN) + 16 * ((col >> 3) ^ (4 * (row & 3))) + 2 * (col & 7));
+                    mk[4 * v4 + 0] = r.x & 0xffffu;
+                    mk[4 * v4 + 1] = r.x >> 16;
+                    mk[4 * v4 + 2] = r.y & 0xffffu;
+                    mk[4 * v4 + 3] = r.y >> 16;
+                }
+            } else {
+#pragma unroll
+                for (int v = 0; v < 16; ++v) mk[v] = p.mask[off + (int64_t)(row0 + 8 * (v >> 2) + (v & 3)) * p.ldo];
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float val = t.acc[i][nt][v] * bf16_to_f32((uint16_t)mk[v]);
+                const int64_t idx = off + (int64_t)(row0 + 8 * (v >> 2) + (v & 3)) * p.ldo;
+                if (OUT_BF16)
+                    store_out(&((uint16_t*)p.out)[idx], f32_to_bf16_rne(val));
+                else
+                    store_out(&((float*)p.out)[idx], val);
+            }
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+template <int TM, int TN, int WR, int WC, int S, int CH, int WPE>
+static void launch_sddmm_tile_t(const SddmmTileArgs& a, bool y_colmajor, bool out_bf16, int grid, hipStream_t stream) {
+    const dim3 g(grid), b(64 * WR * WC);
+    if (y_colmajor) {
+        if (out_bf16)
+            hipLaunchKernelGGL((sddmm_tile_kernel<TM, TN, WR, WC, S, true, true, CH, WPE>), g, b, 0, stream, a);
+        else
+            hipLaunchKernelGGL((sddmm_tile_kernel<TM, TN, WR, WC, S, true, false, CH, WPE>), g, b, 0, stream, a);
+    } else {
+        if (out_bf16)
+            hipLaunchKernelGGL((sddmm_tile_kernel<TM, TN, WR, WC, S, false, true, CH, WPE>), g, b, 0, stream, a);
+        else
+            hipLaunchKernelGGL((sddmm_tile_kernel<TM, TN, WR, WC, S, false, false, CH, WPE>), g, b, 0, stream, a);
+    }
+}
+
+hipError_t launch_sddmm_tile(const SddmmTileArgs& a, const SddmmTileVariant& v, bool y_colmajor, bool out_bf16, int grid,
+                             hipStream_t stream) {
+    if (grid <= 0) return hipSuccess;
+#define BSP_SDDMM_TILE_CASE(TM, TN, WR, WC, S, CH, WPE)                                             \
+    if (v.tile_m == TM && v.tile_n == TN && v.stages == S) {                                       \
+        launch_sddmm_tile_t<TM, TN, WR, WC, S, CH, WPE>(a, y_colmajor, out_bf16, grid, stream);    \
+        return hipGetLastError();                                                                  \
+    }
+    BSP_SDDMM_TILES(BSP_SDDMM_TILE_CASE)
+#undef BSP_SDDMM_TILE_CASE
+    return hipErrorInvalidValue;
+}
+
+}  // namespace bsp

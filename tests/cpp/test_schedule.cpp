@@ -311,6 +311,45 @@ void check_sddmm(const Bsr& m, int64_t K, int cus, const std::string& name) {
     std::printf("%-34s items %5zu chunk %d grid %5zu\n", name.c_str(), s.items.size(), s.chunk, s.wgmap.size());
 }
 
+// SDDMM tiles: every (32-row stripe, column, output offset) of the mask
+// once, items within the tile, the XCDs' shares equal.
+void check_sddmm_tiles(const Bsr& m, int64_t K, int cus, const SddmmTileVariant& v, const std::string& name) {
+    SddmmTiles s;
+    std::string msg;
+    const bsp_bsr_desc d = m.desc();
+    const int st = build_sddmm_tiles(&d, K, cus, v, s, msg);
+    expect(st == BSP_OK, name + ": build " + msg);
+    if (st != BSP_OK) return;
+    std::vector<std::tuple<int64_t, int64_t, int64_t>> want, got;
+    for (int64_t i = 0; i < m.H / m.R; ++i)
+        for (int64_t blk = m.indptr[i]; blk < m.indptr[i + 1]; ++blk)
+            for (int64_t r = 0; r < m.R; r += v.tile_m)
+                for (int64_t c = 0; c < m.C; c += kSub)
+                    want.emplace_back(i * m.R + r, m.indices[blk] * m.C + c, blk * m.R * m.C + r * m.C + c);
+    std::vector<int> used(s.ent_col.size(), 0);
+    bool fits = s.items.size() % kNumXcd == 0 && m.C % s.cb == 0 && v.tile_n % s.cb == 0;
+    std::vector<int> share(kNumXcd, 0);
+    for (size_t g = 0; g < s.items.size(); ++g) {
+        const SddmmItem& it = s.items[g];
+        if (it.e_end <= it.e_begin) continue;
+        ++share[g % kNumXcd];
+        fits = fits && it.e_end - it.e_begin <= v.tile_n / s.cb && it.e_end <= (int32_t)used.size();
+        for (int32_t e = it.e_begin; fits && e < it.e_end; ++e) {
+            ++used[e];
+            for (int64_t c = 0; c < s.cb; c += kSub) got.emplace_back(it.x_row0, s.ent_col[e] + c, s.ent_off[e] + c);
+        }
+    }
+    std::sort(want.begin(), want.end());
+    std::sort(got.begin(), got.end());
+    expect(fits, name + ": items fit the tile");
+    expect(want == got, name + ": every sub-block once, with its column and offset");
+    expect(std::all_of(used.begin(), used.end(), [](int u) { return u == 1; }), name + ": chunks used once");
+    expect(*std::max_element(share.begin(), share.end()) - *std::min_element(share.begin(), share.end()) <=
+               (int)kNumXcd,
+           name + ": XCD shares");
+    std::printf("%-34s items %5d chunk %d grid %5zu\n", name.c_str(), s.n_items, s.cb, s.items.size());
+}
+
 void check_spgemm(const Bsr& a, const Bsr& b, int cus, const std::string& name) {
     SpgemmSchedule s;
     std::string msg;
@@ -617,6 +656,25 @@ int main() {
     check_sddmm(skewed(2048, 2048, 64, 32, 300, 11), 128, cus, "sddmm 64x32 blocks, skewed");
     check_sddmm(uniform(1024, 1024, 128, 128, 20, 12), 64, cus, "sddmm 128x128 blocks");
     check_sddmm(banded(8192, 32, 8, 655, 20), 128, cus, "sddmm banded 8192^2 (column bands)");
+    check_sddmm_tiles(uniform(4096, 4096, 32, 32, 4096, 21), 512, cus, {32, 128, 2}, "sddmm tiles 32x32 25%");
+    check_sddmm_tiles(skewed(2048, 1920, 64, 96, 200, 22), 512, cus, {64, 128, 2}, "sddmm tiles 64x96, skewed");
+    check_sddmm_tiles(uniform(2048, 2048, 128, 64, 100, 23), 512, 16, {32, 128, 4}, "sddmm tiles 128x64 in 32 rows");
+    check_sddmm_tiles(uniform(8192, 8192, 256, 256, 256, 24), 8192, cus, {256, 256, 2}, "sddmm tiles 256x256");
+    check_sddmm_tiles(uniform(512, 512, 64, 512, 2, 25), 96, cus, {64, 128, 3}, "sddmm tiles 64x512");
+    check_sddmm_tiles(uniform(1024, 1024, 32, 32, 0, 9), 512, cus, {32, 128, 2}, "sddmm tiles empty");
+    {
+        // The rule: short K and few blocks stay with the 32-row kernels.
+        auto tile = [&](const Bsr& m, int64_t K) {
+            const bsp_bsr_desc d = m.desc();
+            return sddmm_choose_tile(&d, K, 256).tile_m;
+        };
+        const Bsr few = uniform(1024, 1024, 32, 32, 102, 26), half = uniform(4096, 4096, 64, 64, 1024, 27);
+        expect(tile(few, 320) == 0 && tile(few, 8192) == 0, "sddmm tile rule: few blocks");
+        expect(tile(half, 64) == 0 && tile(half, 96) == 64 && tile(half, 512) == 64, "sddmm tile rule: 64x64 25%");
+        expect(tile(uniform(4096, 4096, 32, 32, 4096, 21), 256) == 0, "sddmm tile rule: 32x32 25% K=256");
+        expect(tile(uniform(4096, 4096, 32, 32, 4096, 21), 288) == 32, "sddmm tile rule: 32x32 25% K=288");
+        expect(tile(uniform(8192, 8192, 256, 256, 256, 24), 8192) == 256, "sddmm tile rule: 256x256 K=8192");
+    }
     check_spgemm(uniform(2048, 2048, 32, 32, 300, 13), uniform(2048, 2048, 32, 32, 300, 14), cus,
                  "spgemm 2048^2 7% x 7%");
     check_spgemm(skewed(1024, 512, 64, 32, 80, 15), uniform(512, 768, 32, 96, 30, 16), cus,

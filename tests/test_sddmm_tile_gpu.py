@@ -1,0 +1,101 @@
+"""The SDDMM tile kernel on the GPU against the oracle: every compiled tile,
+at the edges of its steps (64 of K), tiles and column chunks.
+
+Bound: the kernel and the oracle add the same K products (exact in fp32) in
+fp32 in different orders, so each differs from the exact sum by at most
+K * 2^-24 * sum |x_k y_k| <= K^2 * 2^-24 for |x|, |y| <= 1, and the mask
+product rounds once more; twice that is allowed, and one bf16 rounding (2^-8)
+on bf16 output."""
+import numpy as np
+import pytest
+
+from helpers import W, bsr_of, capi, golden_sddmm, run_sddmm, with_values
+
+pytestmark = pytest.mark.gpu
+
+TILES = ["32,128,2", "32,128,4", "64,128,2", "64,128,3", "128,128,2", "256,256,2"]
+
+
+def _check(got, gold, K, out_dtype, what):
+    assert np.isfinite(got).all(), what
+    err = np.abs(got.astype(np.float64) - gold)
+    bound = 2 * (K * K + 1) * 2.0 ** -24 + (2.0 ** -8 * np.abs(gold) if out_dtype == "bf16" else 0)
+    assert np.all(err <= bound), f"{what}: {err.max()}"
+
+
+def _mask(R, C, seed):
+    """8 R x 1536-column mask, about 30%, with an empty block row, a full one and,
+    out of order, a repeated column."""
+    rng = np.random.default_rng(seed)
+    nbc = 1536 // C
+    cols = [np.sort(rng.choice(nbc, size=max(1, round(0.3 * nbc)), replace=False)) for _ in range(8)]
+    cols[2] = np.zeros(0, np.int64)
+    cols[5] = np.arange(nbc)
+    cols[6] = np.array([nbc - 1, 0, nbc - 1][: max(1, min(3, nbc))])
+    indptr = np.concatenate([[0], np.cumsum([c.size for c in cols])]).astype(np.int32)
+    m = W.BsrArrays(8 * R, nbc * C, R, C, indptr, np.concatenate(cols).astype(np.int32))
+    return with_values(m, "RAND", seed=seed)
+
+
+@pytest.mark.parametrize("tile", TILES)
+@pytest.mark.parametrize("layout", ["row", "col"])
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+def test_tiles_match_oracle(tile, layout, out_dtype, monkeypatch):
+    monkeypatch.setenv("BSP_SDDMM_TILE", tile)
+    tm = int(tile.split(",")[0])
+    # C: one chunk per tile and per block, several chunks per tile (32, 96) and
+    # several per block (256); K: one half step, one step, an odd half, more
+    # steps than the ring is deep.
+    for C, K in ((32, 32), (96, 64), (64, 160), (128, 352), (256, 96)):
+        mask = _mask(tm, C, seed=tm + C)
+        rng = np.random.default_rng(K)
+        x, y = W.dense_content(mask.H, K, "RAND", rng), W.dense_content(K, mask.W, "RAND", rng)
+        print(tile, layout, out_dtype, C, K, flush=True)
+        plan = capi.SddmmPlan(bsr_of(mask), K, capi.ROW_MAJOR if layout == "row" else capi.COL_MAJOR, out_dtype)
+        assert plan.info()["group"] == tm // 32
+        yy = y if layout == "row" else np.ascontiguousarray(y.T)
+        got = run_sddmm(mask, x, yy, out_dtype, y_layout=capi.ROW_MAJOR if layout == "row" else capi.COL_MAJOR,
+                        plan=plan)
+        plan.close()
+        _check(got, golden_sddmm(mask, x, y), K, out_dtype, f"{tile} C={C} K={K} {layout}")
+
+
+@pytest.mark.parametrize("layout", ["row", "col"])
+def test_strides_and_mask_alignment(layout, monkeypatch):
+    """Rows of X and Y strided, the mask two bytes off a 16-byte boundary (then
+    read value by value): the same bits as the packed, aligned call."""
+    import torch
+    monkeypatch.setenv("BSP_SDDMM_TILE", "64,128,2")
+    mask, K = _mask(64, 96, seed=3), 224
+    rng = np.random.default_rng(5)
+    x, y = W.dense_content(mask.H, K, "RAND", rng), W.dense_content(K, mask.W, "RAND", rng)
+    yy = y if layout == "row" else np.ascontiguousarray(y.T)
+    lay = capi.ROW_MAJOR if layout == "row" else capi.COL_MAJOR
+    plan = capi.SddmmPlan(bsr_of(mask), K, lay, "f32")
+    dev = lambda a: torch.from_numpy(np.ascontiguousarray(a).view(np.int16)).cuda()
+    dx, dy, dm = dev(x), dev(yy), dev(mask.data)
+    wide = lambda t, pad: torch.nn.functional.pad(t, (0, pad), value=0x7FC0)
+    off = torch.zeros(dm.numel() + 8, dtype=torch.int16, device="cuda")
+    off[1:dm.numel() + 1] = dm
+    outs = []
+    for m, px, py in ((dm, dx, dy), (off[1:dm.numel() + 1], wide(dx, 24), wide(dy, 8))):
+        out = torch.full((dm.numel(),), float("nan"), device="cuda")
+        plan.run(m, px, py, out, stream=torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        outs.append(out.cpu().numpy())
+    plan.close()
+    np.testing.assert_array_equal(outs[0], outs[1])
+    _check(outs[0], golden_sddmm(mask, x, y), K, "f32", layout)
+
+
+def test_chosen_for_long_k():
+    """K past the one-shot kernel with work for every compute unit takes the
+    tile kernel by itself; the looped kernel (BSP_SDDMM_LOOP) stays."""
+    rng = np.random.default_rng(7)
+    mask = with_values(W.random_positions(2048, 2048, 64, 64, 300, rng), "RAND", seed=1)
+    x, y = W.dense_content(2048, 416, "RAND", rng), W.dense_content(416, 2048, "RAND", rng)
+    plan = capi.SddmmPlan(bsr_of(mask), 416)
+    assert plan.info()["stages"] >= 2 and plan.info()["n_entries"] == 1200
+    got = run_sddmm(mask, x, y, plan=plan)
+    plan.close()
+    _check(got, golden_sddmm(mask, x, y), 416, "f32", "chosen")
