@@ -40,7 +40,7 @@ struct bsp_plan {
     bsp::SpgemmRun* d_runs = nullptr;  // wave runs
     int32_t wg_per_xcd = 0;
     int32_t sddmm_one_shot = 0;  // SDDMM: the one-shot kernel runs this plan
-    int32_t tile = 0;            // SDDMM: the tile kernel runs this plan on tiles of that height
+    int32_t tile = 0;            // SDDMM, SpGEMM: the tile kernel runs this plan on tiles of that height
     bsp::SddmmTileVariant sddmm_tile{};
     int32_t cb_shift = 0;        // SDDMM tiles: log2 of the column chunks' width
     // SpMM persistent kernel: variant, unit records and A words (the B words
@@ -917,8 +917,10 @@ int bsp_spgemm_plan_create(bsp_plan** out, const bsp_bsr_desc* a, const bsp_bsr_
     // first round's tail (8192^2, 5% x 5%: 29.4 -> 28.2 us fp32).
     int rounds = 2;
     if (const char* e = std::getenv("BSP_SPGEMM_ROUNDS")) rounds = std::atoi(e);
+    const int tile = bsp::spgemm_choose_tile(a, b, (int64_t)ix.size(), cus);
     bsp::SpgemmSchedule s;
-    st = bsp::build_spgemm_schedule(a, b, cus, stages, rounds, s, msg);
+    st = tile ? bsp::build_spgemm_tiles(a, b, tile, s, msg)
+              : bsp::build_spgemm_schedule(a, b, cus, stages, rounds, s, msg);
     if (st != BSP_OK) return fail(st, msg);
 
     DeviceGuard g(device);
@@ -938,15 +940,16 @@ int bsp_spgemm_plan_create(bsp_plan** out, const bsp_bsr_desc* a, const bsp_bsr_
     p->out_indptr = std::move(s.indptr);
     p->out_indices = std::move(s.indices);
     bsp_plan_info& info = p->info;
+    p->tile = tile;
     info.kind = 4;
-    info.tile_n = bsp::kSub;
+    info.tile_n = tile ? tile : bsp::kSub;
     info.n_tiles = 1;
-    info.n_items = (int32_t)s.tasks.size();
-    info.n_entries = (int32_t)s.terms.size();
+    info.n_items = (int32_t)s.n_sub_tasks;
+    info.n_entries = (int32_t)s.n_sub_terms;
     info.grid = s.grid;
-    info.max_item_entries = s.max_task_terms;
-    info.stages = stages;
-    info.group = 1;
+    info.max_item_entries = tile ? s.max_task_terms * 2 : s.max_task_terms;
+    info.stages = tile ? 2 : stages;
+    info.group = tile ? tile / bsp::kSub : 1;
     p->wg_per_xcd = s.wg_per_xcd;
     hipError_t e = upload((bsp::SpgemmTask**)&p->d_wgs, s.tasks);
     if (e == hipSuccess) e = upload(&p->d_terms, s.terms);
@@ -979,6 +982,21 @@ int bsp_spgemm(const bsp_plan* p, const uint16_t* a_vals, const uint16_t* b_vals
         return fail(BSP_ERR_INVALID_ARGUMENT, "A, B and output values must be 16-byte aligned");
     DeviceGuard g(p->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
+    if (p->tile) {
+        bsp::SpgemmTileArgs ta{};
+        ta.a = a_vals;
+        ta.b = b_vals;
+        ta.out = out_vals;
+        ta.tasks = (const bsp::SpgemmTask*)p->d_wgs;
+        ta.terms = p->d_terms;
+        ta.lda = (int32_t)p->C;
+        ta.ldb = (int32_t)p->BC;
+        ta.ldo = (int32_t)p->BC;
+        const hipError_t te =
+            bsp::launch_spgemm_tile(ta, p->tile, p->out_dtype == BSP_DTYPE_BF16, p->info.grid, (hipStream_t)stream);
+        if (te != hipSuccess) return hip_fail(te, "SpGEMM launch");
+        return BSP_OK;
+    }
     bsp::SpgemmArgs args{};
     args.a = a_vals;
     args.b = b_vals;

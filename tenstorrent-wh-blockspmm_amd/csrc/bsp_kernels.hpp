@@ -203,6 +203,20 @@ struct SddmmTileArgs {
 hipError_t launch_sddmm_tile(const SddmmTileArgs& a, const SddmmTileVariant& v, bool y_colmajor, bool out_bf16, int grid,
                              hipStream_t stream);
 
+// SpGEMM on tile x tile output tiles (64 or 128; R, C and BC multiples of 64).
+struct SpgemmTileArgs {
+    const uint16_t* a;          // A block values (bf16), R x C blocks
+    const uint16_t* b;          // B block values (bf16), C x BC blocks
+    void* out;                  // C block values (fp32 or bf16), R x BC blocks
+    const SpgemmTask* tasks;    // one per workgroup (empty range: idle)
+    const uint64_t* terms;      // per 64-deep step: A offset / 32 (low 32 bits) | B offset / 32 (high)
+    int32_t lda;                // row stride inside an A block (= C)
+    int32_t ldb;                // row stride inside a B block (= BC)
+    int32_t ldo;                // row stride inside an output block (= BC)
+    int32_t pad;
+};
+hipError_t launch_spgemm_tile(const SpgemmTileArgs& a, int tile, bool out_bf16, int grid, hipStream_t stream);
+
 struct SpgemmArgs {
     const uint16_t* a;          // A block values (bf16), R x C blocks
     const uint16_t* b;          // B block values (bf16), C x BC blocks

@@ -1274,8 +1274,17 @@ int spgemm_symbolic(const bsp_bsr_desc* a, const bsp_bsr_desc* b, std::vector<in
     return BSP_OK;
 }
 
-int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_cus, int stages, int rounds,
-                          SpgemmSchedule& s, std::string& msg) {
+namespace {
+
+// Cost of a task: its products, and its store counted as two.
+int64_t spgemm_task_cost(const SpgemmTask& t) { return (t.t_end - t.t_begin) + 2; }
+
+// The part of a SpGEMM schedule that does not depend on the kernel: structure,
+// tasks of tile x tile outputs and their terms of `deep` steps of the shared
+// dimension, ordered by XCD region (region x's tasks are region_begin[x] ..
+// region_begin[x + 1]).
+int build_spgemm_regions(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int64_t tile, int64_t deep, SpgemmSchedule& s,
+                         std::vector<int32_t>& region_begin, std::vector<int64_t>& region_cost, std::string& msg) {
     int st = check_spgemm_operands(a, b, msg);
     if (st != BSP_OK) return st;
     const int64_t R = a->R, C = a->C, BC = b->C;
@@ -1285,7 +1294,7 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
         return BSP_ERR_UNSUPPORTED;
     }
     const int64_t nbr = a->H / R, nbc = b->W / BC;
-    const int64_t RS = R / kSub, CS = C / kSub, PS = BC / kSub;
+    const int64_t RS = R / tile, CS = C / deep, PS = BC / tile;
     std::vector<int64_t> mark(nbc, -1), pos(nbc);
     std::vector<int32_t> cnt(nbc), cols;
     std::vector<std::pair<int32_t, int32_t>> pairs;
@@ -1298,20 +1307,23 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
                    [&](int32_t j, const std::pair<int32_t, int32_t>* pr, int32_t np) {
                        const int64_t ob = (int64_t)s.indices.size();
                        s.indices.push_back(j);
-                       if ((int64_t)s.terms.size() + (int64_t)np * CS * RS * PS > INT32_MAX) {
+                       // (Limits in 32x32 sub-blocks for every tile size.)
+                       s.n_sub_tasks += (R / kSub) * (BC / kSub);
+                       s.n_sub_terms += (int64_t)np * (C / kSub) * (R / kSub) * (BC / kSub);
+                       if (s.n_sub_terms > INT32_MAX) {
                            too_big = true;
                            return;
                        }
                        for (int64_t ra = 0; ra < RS; ++ra)
                            for (int64_t pb = 0; pb < PS; ++pb) {
                                SpgemmTask t{};
-                               t.out_off = ob * R * BC + ra * kSub * BC + pb * kSub;
+                               t.out_off = ob * R * BC + ra * tile * BC + pb * tile;
                                t.t_begin = (int32_t)s.terms.size();
                                for (int32_t n = 0; n < np; ++n)
                                    for (int64_t cs = 0; cs < CS; ++cs) {
-                                       const uint64_t ao = (uint64_t)pr[n].first * R * C + ra * kSub * C + cs * kSub;
+                                       const uint64_t ao = (uint64_t)pr[n].first * R * C + ra * tile * C + cs * deep;
                                        const uint64_t bo =
-                                           (uint64_t)pr[n].second * C * BC + cs * kSub * BC + pb * kSub;
+                                           (uint64_t)pr[n].second * C * BC + cs * deep * BC + pb * tile;
                                        s.terms.push_back(ao / kSub | (bo / kSub) << 32);
                                    }
                                t.t_end = (int32_t)s.terms.size();
@@ -1324,14 +1336,13 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
         if ((int64_t)s.indices.size() > INT32_MAX) too_big = true;
         s.indptr[i + 1] = (int32_t)s.indices.size();
     }
-    if (too_big || (int64_t)s.tasks.size() > INT32_MAX) {
+    if (too_big || s.n_sub_tasks > INT32_MAX) {
         msg = "product too large for int32 schedule fields";
         return BSP_ERR_UNSUPPORTED;
     }
     s.nblocks = (int64_t)s.indices.size();
     const int64_t ntask = (int64_t)s.tasks.size();
-    if (num_cus <= 0) num_cus = 256;
-    auto cost = [&](const SpgemmTask& t) -> int64_t { return (t.t_end - t.t_begin) + 2; };
+    auto cost = spgemm_task_cost;
     int64_t total = 0;
     for (const SpgemmTask& t : s.tasks) total += cost(t);
 
@@ -1376,8 +1387,9 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
     }
     // Tasks (and their products) reordered by region, output order inside one.
     std::vector<int32_t> region(ntask);
-    std::vector<int64_t> region_cost(kNumXcd, 0);
-    std::vector<int32_t> region_count(kNumXcd + 1, 0);
+    region_cost.assign(kNumXcd, 0);
+    std::vector<int32_t>& region_count = region_begin;
+    region_count.assign(kNumXcd + 1, 0);
     for (int64_t t = 0; t < ntask; ++t) {
         const int g = row_group[task_row[t]];
         region[t] = g * CG + col_group[(size_t)g * nbc + task_col[t]];
@@ -1402,6 +1414,23 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
         s.tasks.swap(tasks);
         s.terms.swap(terms);
     }
+
+    return BSP_OK;
+}
+
+}  // namespace
+
+int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_cus, int stages, int rounds,
+                          SpgemmSchedule& s, std::string& msg) {
+    std::vector<int32_t> region_count;
+    std::vector<int64_t> region_cost;
+    const int st = build_spgemm_regions(a, b, kSub, kSub, s, region_count, region_cost, msg);
+    if (st != BSP_OK) return st;
+    if (num_cus <= 0) num_cus = 256;
+    const int64_t ntask = (int64_t)s.tasks.size();
+    auto cost = spgemm_task_cost;
+    int64_t total = 0;
+    for (const SpgemmTask& t : s.tasks) total += cost(t);
 
     // Wave runs: contiguous task ranges of one region of about equal cost
     // (products, plus the store counted as two products), `rounds` times as
@@ -1439,6 +1468,70 @@ int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_
     s.runs.assign((size_t)s.grid * 4, SpgemmRun{(int32_t)ntask, (int32_t)ntask, pend, pend});
     for (int x = 0; x < kNumXcd; ++x)
         std::copy(region_runs[x].begin(), region_runs[x].end(), s.runs.begin() + (size_t)x * per * 4);
+    return BSP_OK;
+}
+
+// R, C and BC multiples of 64 take tiles: a 32x32 sub-block task loads 4 KB per
+// 65 kFLOP product, a 64 x 64 tile half and a 128 x 128 tile a quarter of that
+// (us of the 32x32 kernel : 64 : 128 tiles; 4096^2, 128 x 128 blocks, bf16 out:
+// 25% 62.0 : 23.2 : 24.6, 50% 225 : 63.1 : 50.4, 12% f32 16.9 : 8.8 : 9.1;
+// 8192^2 25% 625 : 144 : 133; 64 x 64 blocks, 4096^2 25% 60.9 : 25.2; 2% 3.3 :
+// 2.7).  128 x 128 tiles are the better ones with six or more 64-deep steps a
+// tile on average and two tiles per compute unit; shorter lists are all start
+// and store, which more and smaller workgroups overlap better.
+int spgemm_choose_tile(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int64_t out_blocks, int num_cus) {
+    const int64_t forced = env_int("BSP_SPGEMM_TILE", -1);  // 0: the 32x32 kernel, 64 or 128 where the blocks allow it
+    const int64_t R = a->R, C = a->C, BC = b->C;
+    if (forced == 0 || C % 64 || R % 64 || BC % 64 || out_blocks <= 0) return 0;
+    if (R * C >= (int64_t)1 << 30 || C * BC >= (int64_t)1 << 30) return 0;  // 32-bit byte offsets inside a block
+    const bool can128 = R % 128 == 0 && BC % 128 == 0;
+    if (forced > 0) return forced == 128 && can128 ? 128 : 64;
+    if (num_cus <= 0) num_cus = 256;
+    if (!can128 || out_blocks * (R / 128) * (BC / 128) < 2 * (int64_t)num_cus) return 64;
+    int64_t pairs = 0;  // block pairs that meet
+    for (int64_t e = 0; e < a->nblocks; ++e) pairs += b->indptr[a->indices[e] + 1] - b->indptr[a->indices[e]];
+    return pairs * (C / 64) >= 6 * out_blocks ? 128 : 64;
+}
+
+int build_spgemm_tiles(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int tile, SpgemmSchedule& s,
+                       std::string& msg) {
+    std::vector<int32_t> region;
+    std::vector<int64_t> region_cost;
+    const int st = build_spgemm_regions(a, b, tile, 64, s, region, region_cost, msg);
+    if (st != BSP_OK) return st;
+    // Region x's tiles run on XCD x, longest first; what a region's cost is
+    // over the mean goes, shortest tiles first, to the XCDs below it (regions
+    // are cut between block rows and columns, so a few large blocks leave them
+    // up to 15% apart, and an XCD's tiles come in few rounds).
+    std::vector<std::vector<int32_t>> bins(kNumXcd);
+    int64_t total = 0;
+    for (int x = 0; x < kNumXcd; ++x) {
+        total += region_cost[x];
+        for (int32_t t = region[x]; t < region[x + 1]; ++t) bins[x].push_back(t);
+        std::stable_sort(bins[x].begin(), bins[x].end(), [&](int32_t p, int32_t q) {
+            return s.tasks[p].t_end - s.tasks[p].t_begin > s.tasks[q].t_end - s.tasks[q].t_begin;
+        });
+    }
+    for (;;) {
+        const int hi = (int)(std::max_element(region_cost.begin(), region_cost.end()) - region_cost.begin());
+        const int lo = (int)(std::min_element(region_cost.begin(), region_cost.end()) - region_cost.begin());
+        if (bins[hi].empty()) break;
+        const int64_t c = spgemm_task_cost(s.tasks[bins[hi].back()]);
+        if (region_cost[lo] + c > region_cost[hi] - c || region_cost[hi] * kNumXcd <= total) break;
+        bins[lo].push_back(bins[hi].back());
+        bins[hi].pop_back();
+        region_cost[lo] += c;
+        region_cost[hi] -= c;
+    }
+    size_t per = 1;
+    for (const auto& b : bins) per = std::max(per, b.size());
+    std::vector<SpgemmTask> order(per * kNumXcd, SpgemmTask{0, 0, 0});
+    for (int x = 0; x < kNumXcd; ++x)
+        for (size_t j = 0; j < bins[x].size(); ++j) order[j * kNumXcd + x] = s.tasks[bins[x][j]];
+    s.pieces = (int32_t)s.tasks.size();
+    s.tasks.swap(order);
+    s.grid = (int32_t)s.tasks.size();
+    s.wg_per_xcd = (int32_t)per;
     return BSP_OK;
 }
 

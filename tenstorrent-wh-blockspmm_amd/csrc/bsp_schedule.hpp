@@ -363,6 +363,8 @@ static_assert(sizeof(SpgemmRun) == 16, "SpgemmRun layout is shared with the kern
 // 32-column steps of the shared dimension).
 struct SpgemmSchedule {
     int64_t nblocks = 0;             // output blocks
+    int64_t n_sub_tasks = 0;         // 32x32 output sub-blocks
+    int64_t n_sub_terms = 0;         // their 32x32x32 products
     std::vector<int32_t> indptr;     // output block-row pointers (H/R + 1)
     std::vector<int32_t> indices;    // output block columns (nblocks)
     std::vector<SpgemmTask> tasks;   // one per output sub-block, in output order
@@ -389,6 +391,14 @@ int spgemm_symbolic(const bsp_bsr_desc* a, const bsp_bsr_desc* b, std::vector<in
 // a ring of `stages` stages.
 int build_spgemm_schedule(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int num_cus, int stages, int rounds,
                           SpgemmSchedule& s, std::string& msg);
+
+// SpGEMM tiles (spgemm_tile_kernel): the tile size a plan takes (128 or 64, or
+// 0 for the 32x32 kernel), and its schedule: tasks are tile x tile output
+// tiles, one workgroup each, in launch order (`grid` records, idle slots with
+// no terms), terms the 64-deep steps of their block pairs in the golden's
+// order.  R, C and BC multiples of 64, R and BC of `tile`.
+int spgemm_choose_tile(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int64_t out_blocks, int num_cus);
+int build_spgemm_tiles(const bsp_bsr_desc* a, const bsp_bsr_desc* b, int tile, SpgemmSchedule& s, std::string& msg);
 
 // Structural checks of sparse_common/bsr_matrix.hpp:246-252 / :610-616 plus
 // the CSR invariants the golden relies on implicitly.  On failure returns a

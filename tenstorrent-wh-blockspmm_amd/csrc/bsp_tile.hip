@@ -1,7 +1,7 @@
-// Tile kernel: SDDMM with long K or large blocks, each workgroup computing a
-// TM x TN output tile (gfx950).
+// Tile kernels: SDDMM over long K and SpGEMM over blocks of 64 and more, each
+// a workgroup computing a TM x TN output tile (gfx950).
 //
-// A tile is a product of an A panel, TM rows contiguous along k (X rows, rows
+// Both are a product of an A panel, TM rows contiguous along k (X rows, rows
 // of an A block), and a B panel of TN columns, along k in steps of 64.  A step
 // is one stage of an S-stage LDS ring filled by direct global->LDS loads:
 //   - rows contiguous along k ("k-rows": A, and B when it is stored
@@ -20,7 +20,8 @@
 // publishes the next stage, beside its first reads: one barrier per 64-deep
 // step, and no part of a step is reads alone.
 //
-// Reference semantics: sparse_common/bsr_matrix.hpp:816-857.
+// Reference semantics: sparse_common/bsr_matrix.hpp:816-857 (SDDMM), :741-810
+// (SpGEMM).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -398,6 +399,69 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void sddmm_tile_kernel(SddmmTile
 }
 
 // ---------------------------------------------------------------------------
+// SpGEMM over blocks of 64 and more: a workgroup computes one TM x TN tile of
+// an output block; its terms are the 64-deep steps of the block pairs that
+// meet there, in the golden's order.
+//
+// What bounds it: L2 fills and output stores; most lists are a few steps (4096^2,
+// 128 x 128 blocks, 25%: 4.6 on average, 54 MB read into the L2s and 40 MB
+// written in 20 us; 55 -> 23 us a pass against the 32x32 kernel).  Measured and
+// left out there: a workgroup streaming several tiles through one ring of
+// 32-deep steps (22.3-25.5), eight and sixteen waves (22.8-23.4), bf16 rows
+// gathered in LDS and stored as whole lines (24.6).
+template <int TM, int TN, int WR, int WC, int S, bool OUT_BF16, int WPE>
+__global__ __launch_bounds__(64 * WR * WC, WPE) void spgemm_tile_kernel(SpgemmTileArgs p) {
+    using namespace tile_detail;
+    using T = Tile<TM, TN, WR, WC, S, false>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[T::LDS];
+    const SpgemmTask task = load_const(p.tasks + blockIdx.x);
+    const int n = task.t_end - task.t_begin;
+    if (n <= 0) return;  // idle slot (uniform)
+    T t(smem);
+    // Terms in lanes: lane j has term 64c + j of the current chunk c.
+    const uint64_t* terms = p.terms + task.t_begin;
+    uint32_t lo = 0, hi = 0;
+    auto fetch = [&](int base) {
+        if (base + t.lane < n) {
+            const uint64_t w = terms[base + t.lane];
+            lo = (uint32_t)w;
+            hi = (uint32_t)(w >> 32);
+        }
+        __asm__ volatile("" : "+v"(lo), "+v"(hi));
+    };
+    fetch(0);
+    uint32_t av[T::AL], bv[T::BL];  // byte offsets within a block (blocks are below 4 GB, checked by the plan)
+#pragma unroll
+    for (int j = 0; j < T::AL; ++j)
+        av[j] = 2u * (uint32_t)(t.krow(j, T::AL) * p.lda + 8 * t.kchunk(j, T::AL));
+#pragma unroll
+    for (int j = 0; j < T::BL; ++j) bv[j] = 2u * (uint32_t)(t.nrow(j) * p.ldb + 8 * t.nchunk(j));
+    auto issue = [&](int k, int stage) {
+        if ((k & 63) == 0 && k > 0) fetch(k);
+        const uint16_t* a = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(lo, k & 63) * 32;
+        const uint16_t* b = p.b + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k & 63) * 32;
+#pragma unroll
+        for (int j = 0; j < T::AL; ++j) gl_lds16_s(av[j], a, t.a_lds(stage, j));
+#pragma unroll
+        for (int j = 0; j < T::BL; ++j) gl_lds16_s(bv[j], b, t.b_lds(stage, j));
+    };
+    t.run(n, false, true, issue);
+#pragma unroll
+    for (int i = 0; i < T::FM; ++i)
+#pragma unroll
+        for (int nt = 0; nt < T::FN; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int row = (t.wr * T::FM + i) * 32 + 8 * (v >> 2) + 4 * t.q + (v & 3);
+                const int64_t idx = task.out_off + (int64_t)row * p.ldo + (t.wc * T::FN + nt) * 32 + t.l32;
+                if (OUT_BF16)
+                    store_out(&((uint16_t*)p.out)[idx], f32_to_bf16_rne(t.acc[i][nt][v]));
+                else
+                    store_out(&((float*)p.out)[idx], t.acc[i][nt][v]);
+            }
+}
+
+// ---------------------------------------------------------------------------
 template <int TM, int TN, int WR, int WC, int S, int CH, int WPE>
 static void launch_sddmm_tile_t(const SddmmTileArgs& a, bool y_colmajor, bool out_bf16, int grid, hipStream_t stream) {
     const dim3 g(grid), b(64 * WR * WC);
@@ -425,6 +489,25 @@ hipError_t launch_sddmm_tile(const SddmmTileArgs& a, const SddmmTileVariant& v, 
     BSP_SDDMM_TILES(BSP_SDDMM_TILE_CASE)
 #undef BSP_SDDMM_TILE_CASE
     return hipErrorInvalidValue;
+}
+
+template <int TM, int TN, int WR, int WC, int S, int WPE>
+static void launch_spgemm_tile_t(const SpgemmTileArgs& a, bool out_bf16, int grid, hipStream_t stream) {
+    const dim3 g(grid), b(64 * WR * WC);
+    if (out_bf16)
+        hipLaunchKernelGGL((spgemm_tile_kernel<TM, TN, WR, WC, S, true, WPE>), g, b, 0, stream, a);
+    else
+        hipLaunchKernelGGL((spgemm_tile_kernel<TM, TN, WR, WC, S, false, WPE>), g, b, 0, stream, a);
+}
+
+hipError_t launch_spgemm_tile(const SpgemmTileArgs& a, int tile, bool out_bf16, int grid, hipStream_t stream) {
+    if (grid <= 0) return hipSuccess;
+    switch (tile) {
+        case 64: launch_spgemm_tile_t<64, 64, 2, 2, 2, 4>(a, out_bf16, grid, stream); break;
+        case 128: launch_spgemm_tile_t<128, 128, 2, 2, 2, 2>(a, out_bf16, grid, stream); break;
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 }  // namespace bsp

@@ -611,6 +611,52 @@ void check_spmm_stream_pairs(const Bsr& a, int64_t N, int cus, const std::string
                 (long long)w, s.wgs.size());
 }
 
+// SpGEMM tiles: per tile of every output block, its terms -- the 64-deep
+// steps of the (A block, B block) pairs in A's then B's CSR order -- once.
+void check_spgemm_tiles(const Bsr& a, const Bsr& b, int tile, const std::string& name) {
+    SpgemmSchedule s;
+    std::string msg;
+    const bsp_bsr_desc da = a.desc(), db = b.desc();
+    const int st = build_spgemm_tiles(&da, &db, tile, s, msg);
+    expect(st == BSP_OK, name + ": build " + msg);
+    if (st != BSP_OK) return;
+    const int64_t R = a.R, C = a.C, BC = b.C;
+    std::map<int64_t, std::vector<uint64_t>> want, got;  // by output offset
+    int64_t nblocks = 0;
+    for (int64_t i = 0; i < a.H / R; ++i) {
+        std::map<int32_t, std::vector<std::pair<int64_t, int64_t>>> row;
+        for (int32_t ai = a.indptr[i]; ai < a.indptr[i + 1]; ++ai)
+            for (int32_t bi = b.indptr[a.indices[ai]]; bi < b.indptr[a.indices[ai] + 1]; ++bi)
+                row[b.indices[bi]].push_back({ai, bi});
+        for (const auto& [j, pairs] : row) {
+            for (int64_t r = 0; r < R; r += tile)
+                for (int64_t c = 0; c < BC; c += tile)
+                    for (const auto& [ai, bi] : pairs)
+                        for (int64_t k = 0; k < C; k += 64)
+                            want[nblocks * R * BC + r * BC + c].push_back(
+                                (uint64_t)(ai * R * C + r * C + k) / 32 |
+                                (uint64_t)(bi * C * BC + k * BC + c) / 32 << 32);
+            ++nblocks;
+        }
+    }
+    size_t tiles = 0;
+    std::vector<int64_t> share(kNumXcd, 0);
+    for (size_t g = 0; g < s.tasks.size(); ++g) {
+        const SpgemmTask& t = s.tasks[g];
+        if (t.t_end <= t.t_begin) continue;
+        ++tiles;
+        share[g % kNumXcd] += t.t_end - t.t_begin + 2;
+        got[t.out_off] = {s.terms.begin() + t.t_begin, s.terms.begin() + t.t_end};
+    }
+    expect(tiles == want.size() && s.nblocks == nblocks, name + ": tile count");
+    expect(got == want, name + ": terms of every tile");
+    expect(s.n_sub_tasks == nblocks * (R / 32) * (BC / 32), name + ": sub-block count");
+    expect(s.tasks.size() % kNumXcd == 0 && s.grid == (int32_t)s.tasks.size(), name + ": grid");
+    std::printf("%-34s tiles %5zu grid %5zu XCD cost %lld..%lld\n", name.c_str(), tiles, s.tasks.size(),
+                (long long)*std::min_element(share.begin(), share.end()),
+                (long long)*std::max_element(share.begin(), share.end()));
+}
+
 int main() {
     const int cus = 256;
     check_pairing();
@@ -681,6 +727,23 @@ int main() {
                  "spgemm 64x32 x 32x96, duplicates");
     check_spgemm(uniform(512, 512, 128, 128, 6, 17), uniform(512, 256, 128, 64, 5, 18), cus,
                  "spgemm 128x128 x 128x64");
+    check_spgemm_tiles(uniform(4096, 4096, 128, 128, 256, 31), uniform(4096, 4096, 128, 128, 256, 32), 128,
+                       "spgemm tiles 128 of 128x128 25%");
+    check_spgemm_tiles(uniform(2048, 1024, 128, 64, 120, 33), uniform(1024, 1536, 64, 192, 60, 34), 64,
+                       "spgemm tiles 64 of 128x64 x 64x192");
+    check_spgemm_tiles(skewed(1024, 1024, 64, 64, 60, 35), uniform(1024, 512, 64, 64, 30, 36), 64,
+                       "spgemm tiles 64, skewed, duplicates");
+    {
+        auto tile = [&](int64_t R, int64_t C, int64_t BC, int64_t na, int64_t nb, int64_t out) {
+            const Bsr a = uniform(4096, 4096, R, C, na, 37), b = uniform(4096, 4096, C, BC, nb, 38);
+            const bsp_bsr_desc da = a.desc(), db = b.desc();
+            return spgemm_choose_tile(&da, &db, out, 256);
+        };
+        expect(tile(32, 64, 64, 800, 400, 1000) == 0 && tile(64, 32, 64, 800, 800, 1000) == 0, "spgemm tile rule: 32");
+        expect(tile(64, 64, 64, 400, 400, 1000) == 64 && tile(128, 128, 128, 512, 512, 1024) == 128 &&
+                   tile(128, 128, 128, 256, 256, 900) == 64 && tile(256, 64, 128, 100, 100, 50) == 64,
+               "spgemm tile rule: 64 and 128");
+    }
     std::printf("%s (%d failed checks)\n", g_fail ? "FAIL" : "PASS", g_fail);
     return g_fail ? 1 : 0;
 }

@@ -1,0 +1,58 @@
+"""The SpGEMM tile kernel on the GPU against the oracle, at the edges of its
+tiles, of its ring (one step a tile, and more than two) and of the 64 terms it
+holds in registers.
+
+Bound: products of bf16 values are exact in fp32 and both sides add the same n
+of them in fp32, in different orders: each differs from the exact sum by at
+most n * 2^-24 * sum |a b| <= n^2 * 2^-24 for |a|, |b| <= 1; twice that is
+allowed, and one bf16 rounding (2^-8) on bf16 output."""
+import numpy as np
+import pytest
+
+from helpers import W, bsr_of, capi, golden_spgemm, run_spgemm, spgemm_k_eff, with_values
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(a, b, out_dtype, tile=None):
+    plan = capi.SpgemmPlan(bsr_of(a), bsr_of(b), out_dtype)
+    if tile is not None:
+        assert plan.info()["tile_n"] == tile
+    st, got = run_spgemm(a, b, out_dtype, plan=plan)
+    plan.close()
+    ip, ix, gold = golden_spgemm(a, b)
+    np.testing.assert_array_equal(st.indptr, ip)
+    np.testing.assert_array_equal(st.indices, ix)
+    n = spgemm_k_eff(a, b, st).astype(np.float64)
+    err = np.abs(got.astype(np.float64) - gold)
+    bound = 2 * (n * n + 1) * 2.0 ** -24 + (2.0 ** -8 * np.abs(gold) if out_dtype == "bf16" else 0)
+    assert np.isfinite(got).all() and np.all(err <= bound), err.max()
+
+
+def _rand(H, Wd, R, C, density, seed):
+    rng = np.random.default_rng(seed)
+    n = max(1, round(density * (H // R) * (Wd // C)))
+    return with_values(W.random_positions(H, Wd, R, C, n, rng), "RAND", seed=seed)
+
+
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("tile,R,C,BC,n,density", [
+    (64, 64, 64, 64, 640, 0.3), (64, 128, 64, 192, 768, 0.3), (64, 64, 128, 64, 512, 1.0),
+    (128, 128, 64, 128, 512, 0.3), (128, 128, 64, 128, 768, 1.0), (128, 256, 256, 128, 1024, 0.4),
+    (128, 128, 192, 384, 1152, 0.5), (64, 64, 64, 64, 4160, 0.06)])
+def test_tiles_match_oracle(tile, R, C, BC, n, density, out_dtype, monkeypatch):
+    monkeypatch.setenv("BSP_SPGEMM_TILE", str(tile))
+    K = -(-n // C) * C
+    a = _rand(-(-n // R) * R // (8 if n > 4000 else 1) // R * R, K, R, C, density, 3)
+    b = _rand(K, -(-n // BC) * BC // (8 if n > 4000 else 1) // BC * BC, C, BC, density, 4)
+    print(tile, R, C, BC, n, density, out_dtype, flush=True)
+    _check(a, b, out_dtype, tile)
+
+
+def test_long_lists():
+    """One output tile with more than 64 terms (the registers' chunk) in a ring
+    of two stages; duplicates and unsorted columns count once per copy."""
+    a = W.BsrArrays(64, 64 * 70, 64, 64, np.array([0, 70], np.int32),
+                    np.concatenate([np.arange(2, 70)[::-1], [3, 3]]).astype(np.int32))
+    b = W.BsrArrays(64 * 70, 64, 64, 64, np.arange(71, dtype=np.int32), np.zeros(70, np.int32))
+    _check(with_values(a, "RAND", seed=5), with_values(b, "RAND", seed=6), "f32", 64)
