@@ -80,13 +80,17 @@ int hip_fail(hipError_t e, const char* what) {
 // Makes `device` current for the lifetime of the guard.
 struct DeviceGuard {
     int prev = -1;
+    bool changed = false;
     hipError_t err = hipSuccess;
     explicit DeviceGuard(int device) {
         err = hipGetDevice(&prev);
-        if (err == hipSuccess && prev != device) err = hipSetDevice(device);
+        if (err == hipSuccess && prev != device) {
+            changed = true;
+            err = hipSetDevice(device);
+        }
     }
     ~DeviceGuard() {
-        if (prev >= 0) (void)hipSetDevice(prev);
+        if (changed) (void)hipSetDevice(prev);
     }
 };
 
