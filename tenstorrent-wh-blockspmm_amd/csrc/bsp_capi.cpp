@@ -362,14 +362,18 @@ bool choose_spmm_sweep(const bsp_bsr_desc* a, int64_t N, int cus) {
 // Whether an SpMM plan runs the persistent kernel, and which variant.  It
 // takes blocks whose stripes do not form row groups (row groups share each B
 // panel among the stripes of a block row, which the per-item group kernels
-// exploit) and N a multiple of 128.  BSP_SPMM_STREAM=0 turns it off;
+// exploit) and N of at least 128 (multiples of 32: the last tile of an N that
+// is no multiple of 128 overlaps the one before and stores its own columns
+// only; against the per-item kernel, 4096^2 25%, N = 160 / 480 / 1056: 10.7 /
+// 14.4 / 32.9 us).  BSP_SPMM_STREAM=0 turns it off;
 // BSP_SPMM_STREAM_VARIANT="tile,sb,sa,nbw[,pipes[,entries per step]]" picks
 // another compiled variant and BSP_SPMM_STREAM_WPC the workgroups per compute
 // unit (all read here, at plan creation).  A two-pipeline variant runs one
 // workgroup per compute unit.
 bool choose_spmm_stream(const bsp_bsr_desc* a, int64_t N, int cus, SpmmStreamVariant* sv, int* wpc) {
     if (env_int("BSP_SPMM_STREAM", 1) == 0) return false;
-    if (N % 128 != 0) return false;
+    if (N < 128 || N % bsp::kSub != 0) return false;
+    const int64_t tiles128 = (N + 127) / 128;
     const int64_t group = env_int("BSP_SPMM_GROUP", bsp::spmm_choose_group(a->R, a->H, N, cus));
     if (group > 1 && (a->R / bsp::kSub) % group == 0) return false;
     bsp::SpmmStreamVariant v = bsp::kSpmmStreamDefault;
@@ -392,12 +396,12 @@ bool choose_spmm_stream(const bsp_bsr_desc* a, int64_t N, int cus, SpmmStreamVar
     // 1024 of them, and only when the pairs could fill the compute units.)
     const int64_t pairs_mode = env_int("BSP_SPMM_PAIRS", 1);
     bool pairs_ok = false;
-    const int64_t pair_units = (a->H / bsp::kSub + 1) / 2 * (N / 128);
-    if (pairs_mode > 0 && N % 128 == 0 && (pairs_mode == 2 || pair_units >= (int64_t)cus)) {
+    const int64_t pair_units = (a->H / bsp::kSub + 1) / 2 * tiles128;
+    if (pairs_mode > 0 && (pairs_mode == 2 || pair_units >= (int64_t)cus)) {
         std::vector<std::pair<int32_t, int32_t>> pl;
         int64_t shared = 0, max_union = 0;
         if (bsp::spmm_stripe_pairs(a, bsp::kPairMaxRows, pl, &shared, &max_union)) {
-            const double tiles = (double)(N / 128), nb = (double)a->nblocks;
+            const double tiles = (double)tiles128, nb = (double)a->nblocks;
             const double uni = nb - (double)shared;  // union entries over all pairs
             int64_t longest = 0;
             for (int64_t i = 0; i < a->H / bsp::kSub; ++i)
@@ -416,7 +420,7 @@ bool choose_spmm_stream(const bsp_bsr_desc* a, int64_t N, int cus, SpmmStreamVar
         if (got < 5) w.pipes = 1;
         if (got < 6) w.eps = 1;
         if (got < 7) w.sr = 1;
-        if (got >= 4 && bsp::spmm_stream_variant_supported(w) && N % w.tile_n == 0 && (w.sr == 1 || pairs_ok)) v = w;
+        if (got >= 4 && bsp::spmm_stream_variant_supported(w) && (w.tile_n == 128 ? w.pipes == 1 || N % 128 == 0 : N % w.tile_n == 0) && (w.sr == 1 || pairs_ok)) v = w;
     }
     int w = -1;
     if (!forced && pairs_ok) {
@@ -432,7 +436,7 @@ bool choose_spmm_stream(const bsp_bsr_desc* a, int64_t N, int cus, SpmmStreamVar
     // as at uniform 1-50%, two workgroups stay faster: 25% 14.2 against 16.0
     // us.)
     if (!forced && !pairs_ok && a->R == bsp::kSub) {
-        const int64_t n_tiles = N / 128, stripes = a->H / bsp::kSub;
+        const int64_t n_tiles = tiles128, stripes = a->H / bsp::kSub;
         int64_t longest = 0;
         for (int64_t i = 0; i < a->H / a->R; ++i) longest = std::max<int64_t>(longest, a->indptr[i + 1] - a->indptr[i]);
         longest *= a->C / bsp::kSub;

@@ -1169,10 +1169,11 @@ __global__ __launch_bounds__(64 * (4 * SR + 1 + NBW) * PIPES) void spmm_stream_k
         if (BSP_SKIP(p, kSkipWrite)) return;
         const int32_t stripe = half == 0 ? un.row : un.aux;
         if (SR > 1 && stripe < 0) return;
+        if (NTW == 1 && wc < (un.n0 & 31)) return;  // columns of the tile before this one
         const int64_t row0 = (int64_t)stripe * 32;
 #pragma unroll
         for (int nt = 0; nt < NTW; ++nt) {
-            const int64_t col = un.n0 + wc * (NTW * 32) + nt * 32 + l32;
+            const int64_t col = (un.n0 & ~31) + wc * (NTW * 32) + nt * 32 + l32;
 #pragma unroll
             for (int v = 0; v < 16; ++v) {
                 const int64_t row = row0 + 8 * (v >> 2) + 4 * q + (v & 3);

@@ -489,8 +489,8 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
         msg = "stream tile must be 128 or 256 columns";
         return BSP_ERR_UNSUPPORTED;
     }
-    if (N <= 0 || N % tile_n != 0 || N > INT32_MAX / 2) {
-        msg = "N must be a positive multiple of the stream tile";
+    if (N < tile_n || (tile_n == 128 ? N % kSub : N % tile_n) != 0 || N > INT32_MAX / 2) {
+        msg = "N must be a multiple of the stream tile, or of 32 and at least 128 with 128-column tiles";
         return BSP_ERR_UNSUPPORTED;
     }
     if (a->R % kSub || a->C % kSub) {
@@ -515,7 +515,11 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
     const int64_t RS = a->R / kSub, CS = a->C / kSub;
     // The scheduled rows: stripes, or stripe pairs (row = the pair's index).
     const int64_t nsr = pairs ? (int64_t)pair_list.size() : a->H / kSub;
-    const int64_t n_tiles = N / tile_n;
+    const int64_t n_tiles = (N + tile_n - 1) / tile_n;
+    const int32_t skip = (int32_t)((n_tiles * tile_n - N) / kSub);  // 32-column parts the last tile shares
+    auto unit_n0 = [&](int64_t t) {
+        return t + 1 < n_tiles || !skip ? (int32_t)(t * tile_n) : (int32_t)(N - tile_n) | skip;
+    };
     const int64_t per_stripe_total = a->nblocks * CS;  // entries summed over one stripe of every block row
     if (per_stripe_total * RS * n_tiles > INT32_MAX - kStreamPad || nsr > INT32_MAX || a->W > INT32_MAX ||
         a->nblocks * a->R * a->C / kSub > UINT32_MAX) {
@@ -529,12 +533,19 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
     s.pairs = pairs ? 1 : 0;
 
     // Column groups: the fewest (1, 2, 4, 8) that bring one XCD's slice of B
-    // to at most 2 MiB, limited by the tile count (or as asked).
+    // to at most 2 MiB, limited by the tile count (or as asked).  Tiles past
+    // the last whole set of groups are spread: each XCD of a row group takes
+    // every cg-th of its stripes there.  A count that leaves more than 3/10 of
+    // the tiles to spread is halved (us, counts 8 / 4 / 2 / 1 of N = 1152, 9
+    // tiles: 26.0 / - / - / 34.2 on 4096^2 25%, 40.4 / - / - / 63.7 on 8192^2
+    // 10%; N = 1536, 12 tiles: 35.1 / 29.8, 67.8 / 61.6; N = 1280, 10 tiles:
+    // 28.1 / - / 29.2, 49.5 / - / 62.3).  Two pipelines: only divisors.
     int64_t cg = 1;
     const int64_t b_bytes = a->W * N * 2;
-    while (cg < kNumXcd && b_bytes / cg > (2 << 20) && n_tiles % (cg * 2) == 0) cg *= 2;
+    while (cg < kNumXcd && b_bytes / cg > (2 << 20) && n_tiles >= cg * 2) cg *= 2;
+    while (pipes == 2 ? n_tiles % cg != 0 : 10 * (n_tiles % cg) > 3 * n_tiles) cg /= 2;
     if (col_groups > 0) cg = col_groups;
-    if (cg < 1 || kNumXcd % cg != 0 || n_tiles % cg != 0) cg = 1;
+    if (cg < 1 || kNumXcd % cg != 0 || (col_groups > 0 && n_tiles % cg != 0)) cg = 1;
     s.col_groups = (int32_t)cg;
     const int64_t rg_count = kNumXcd / cg, tpg = n_tiles / cg;
     const bool rotate = pipes == 1 && env_int("BSP_SPMM_ROTATE", 1) != 0;
@@ -625,14 +636,16 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
         for (int64_t c = 0; c < cg; ++c) {
             const int x = (int)(rg * cg + c);
             std::vector<SpmmStreamUnit> us;
-            for (int32_t sr : rows[rg])  // rows[rg] is longest first
-                for (int64_t t = c * tpg; t < (c + 1) * tpg; ++t) {
-                    if (pairs)
-                        us.push_back({pair_list[sr].first, (int32_t)(t * tile_n), (int32_t)cnt[sr],
-                                      pair_list[sr].second});
-                    else
-                        us.push_back({sr, (int32_t)(t * tile_n), (int32_t)cnt[sr], 0});
-                }
+            for (size_t i = 0; i < rows[rg].size(); ++i) {  // rows[rg] is longest first
+                const int32_t sr = rows[rg][i];
+                auto unit = [&](int64_t t) {
+                    us.push_back({pairs ? pair_list[sr].first : sr, unit_n0(t), (int32_t)cnt[sr],
+                                  pairs ? pair_list[sr].second : 0});
+                };
+                for (int64_t t = c * tpg; t < (c + 1) * tpg; ++t) unit(t);
+                if ((int64_t)i % cg == c)
+                    for (int64_t t = cg * tpg; t < n_tiles; ++t) unit(t);
+            }
             std::vector<std::vector<SpmmStreamUnit>> per_cu, per_wg;
             lpt(us, cus_per_xcd, per_cu);
             for (int cu = 0; cu < cus_per_xcd; ++cu) {
@@ -681,7 +694,8 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
     // the unit's entries at `first`.
     auto rotation = [&](size_t first, int32_t n0) -> int64_t {
         if (!rotate) return 0;
-        const int64_t kcol = spmm_stream_rotation_column(a->W / a->C, (n0 / tile_n) / tpg, cg);
+        // (A spread tile's group is cg: no rotation.)
+        const int64_t kcol = spmm_stream_rotation_column(a->W / a->C, stream_unit_tile(n0, tile_n) / tpg, cg);
         const int64_t len = (int64_t)(s.bw.size() - first);
         int64_t off = 0;
         while (off < len && (int64_t)((uint32_t)s.bw[first + off] / a->C) < kcol) ++off;
@@ -699,7 +713,7 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
                 merge(pt.u.row, pt.u.aux, [&](int32_t col, int64_t k0, int64_t k1) {
                     const uint64_t w0 = k0 >= 0 ? (uint64_t)(k0 * a->R * a->C / kSub) : kNoBlock;
                     const uint64_t w1 = k1 >= 0 ? (uint64_t)(k1 * a->R * a->C / kSub) : kNoBlock;
-                    s.bw.push_back((int64_t)col * a->C | ((int64_t)pt.u.n0 << 32));
+                    s.bw.push_back((int64_t)col * a->C | ((int64_t)(pt.u.n0 & ~(kSub - 1)) << 32));
                     s.apw.push_back(w0 | w1 << 32);
                 });
                 const int64_t off = rotation(first, pt.u.n0);
@@ -714,7 +728,7 @@ int build_spmm_stream(const bsp_bsr_desc* a, int64_t N, int num_cus, int tile_n,
                 for (int64_t t = 0; t < CS; ++t, ++e) {
                     if (e < pt.e0 || e >= pt.e1) continue;
                     const int64_t brow = (int64_t)a->indices[blk] * a->C + kSub * t;
-                    s.bw.push_back(brow | ((int64_t)pt.u.n0 << 32));
+                    s.bw.push_back(brow | ((int64_t)(pt.u.n0 & ~(kSub - 1)) << 32));
                     s.aw.push_back((uint32_t)((blk * a->R * a->C + kSub * sub * a->C + kSub * t) / kSub));
                 }
             const int64_t off = rotation(first, pt.u.n0);

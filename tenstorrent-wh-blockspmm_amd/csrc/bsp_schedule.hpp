@@ -88,13 +88,19 @@ static_assert(sizeof(SpmmStreamWg) == 16, "SpmmStreamWg layout is shared with th
 
 struct SpmmStreamUnit {
     int32_t row;    // stripe (32 output rows)
-    int32_t n0;     // first output column
+    int32_t n0;     // first output column (a multiple of 32) | 32-column parts of the tile that are not stored
+                    // (the last tile of an N that is no multiple of 128 lies at N - 128, over the one before)
     int32_t count;  // entries (0: the stripe has no nonzeros; its tile is stored as zeros)
     int32_t aux;    // one stripe: 0 = store the tile; two pipelines: 1 = this part
                     // goes to the exchange buffer, 2 = add the exchange buffer,
                     // then store.  Stripe pairs: the second stripe (-1: none)
 };
 static_assert(sizeof(SpmmStreamUnit) == 16, "SpmmStreamUnit layout is shared with the kernels");
+
+// Index of the tile that a unit's n0 field names.
+inline int64_t stream_unit_tile(int32_t n0, int tile_n) {
+    return ((n0 & ~(kSub - 1)) + kSub * (n0 & (kSub - 1))) / tile_n;
+}
 
 // Trailing words and units past the last workgroup's stream: the kernels
 // prefetch a few records ahead without a bounds test.
@@ -156,8 +162,8 @@ bool spmm_stripe_pairs(const bsp_bsr_desc* a, int64_t max_rows, std::vector<std:
 constexpr int64_t kPairMaxRows = 1024;
 
 // Persistent schedule for 32-row stripes (any R, C multiples of 32) and
-// tiles of tile_n (128 or 256) columns, N a multiple of tile_n, wg_per_cu
-// workgroups per compute unit.  Units are spread over the XCDs in a 2-D split
+// tiles of tile_n (128 or 256) columns, N a multiple of tile_n (128-column
+// tiles: of 32, and at least 128), wg_per_cu workgroups per compute unit.  Units are spread over the XCDs in a 2-D split
 // (column groups of tiles, row groups of stripes, as xcd_tile_map) and, inside
 // an XCD, longest first onto the least-loaded workgroup.  Cost of a unit:
 // entries + store_cost.

@@ -311,6 +311,66 @@ void check_sddmm(const Bsr& m, int64_t K, int cus, const std::string& name) {
     std::printf("%-34s items %5zu chunk %d grid %5zu\n", name.c_str(), s.items.size(), s.chunk, s.wgmap.size());
 }
 
+// Persistent schedule of an N that leaves a partial last tile or tiles past
+// the column groups: every 32 output columns of every stripe stored once, from
+// a slice of B inside N, with the stripe's entries (rotated by its column
+// group) and the XCDs' entries about equal.
+void check_spmm_stream_ragged(const Bsr& a, int64_t N, int cus, bool pairs, const std::string& name) {
+    SpmmStream s;
+    std::string msg;
+    const bsp_bsr_desc d = a.desc();
+    const int st = build_spmm_stream(&d, N, cus, 128, pairs ? 1 : 2, s, msg, 0, 1, pairs);
+    expect(st == BSP_OK, name + ": build (" + msg + ")");
+    if (st != BSP_OK) return;
+    const int64_t RS = a.R / kSub, CS = a.C / kSub, nsr = a.H / kSub, parts = N / kSub;
+    std::vector<int> stored(nsr * parts, 0);
+    std::vector<int64_t> load(kNumXcd, 0);
+    bool inside = true, words = true;
+    for (size_t g = 0; g < s.wgs.size(); ++g) {
+        const SpmmStreamWg& wg = s.wgs[g];
+        int64_t e = wg.w_begin;
+        load[g % kNumXcd] += wg.n + 2 * wg.n_units;
+        for (int32_t j = 0; j < wg.n_units; ++j) {
+            const SpmmStreamUnit& un = s.units[wg.u_begin + j];
+            const int64_t n0 = un.n0 & ~31, skip = un.n0 & 31;
+            inside = inside && n0 % kSub == 0 && n0 + 128 <= N && skip < 4;
+            for (int64_t part = skip; inside && part < 4; ++part) {
+                ++stored[un.row * parts + n0 / kSub + part];
+                if (pairs && un.aux >= 0) ++stored[un.aux * parts + n0 / kSub + part];
+            }
+            std::multiset<std::pair<int64_t, int64_t>> want, got;  // (B row, A offset)
+            for (int64_t row : {(int64_t)un.row, pairs ? (int64_t)un.aux : (int64_t)-1}) {
+                if (row < 0) continue;
+                const int64_t i = row / RS, sub = row % RS;
+                for (int64_t blk = a.indptr[i]; blk < a.indptr[i + 1]; ++blk)
+                    for (int64_t t = 0; t < CS; ++t)
+                        want.insert({(int64_t)a.indices[blk] * a.C + kSub * t,
+                                     blk * a.R * a.C + kSub * sub * a.C + kSub * t});
+            }
+            for (int32_t k = 0; k < un.count; ++k, ++e) {
+                words = words && (s.bw[e] >> 32) == n0;
+                if (!pairs) {
+                    got.insert({s.bw[e] & 0xffffffffLL, (int64_t)s.aw[e] * kSub});
+                } else {
+                    for (const uint32_t w : {(uint32_t)s.apw[e], (uint32_t)(s.apw[e] >> 32)})
+                        if (w != kNoBlock) got.insert({s.bw[e] & 0xffffffffLL, (int64_t)w * kSub});
+                }
+            }
+            words = words && got == want;
+        }
+        words = words && e == wg.w_begin + wg.n;
+    }
+    expect(inside, name + ": tiles inside N");
+    expect(words, name + ": entries of every unit");
+    expect(std::all_of(stored.begin(), stored.end(), [](int v) { return v == 1; }), name + ": columns stored once");
+    const int64_t most = *std::max_element(load.begin(), load.end());
+    int64_t total = 0;
+    for (int64_t l : load) total += l;
+    expect(most * kNumXcd <= total + total / 4 + 800, name + ": XCD loads");
+    std::printf("%-34s cg %d tiles %d XCD load %lld of mean %lld\n", name.c_str(), s.col_groups, s.n_tiles,
+                (long long)most, (long long)(total / kNumXcd));
+}
+
 // SDDMM tiles: every (32-row stripe, column, output offset) of the mask
 // once, items within the tile, the XCDs' shares equal.
 void check_sddmm_tiles(const Bsr& m, int64_t K, int cus, const SddmmTileVariant& v, const std::string& name) {
@@ -702,6 +762,12 @@ int main() {
     check_sddmm(skewed(2048, 2048, 64, 32, 300, 11), 128, cus, "sddmm 64x32 blocks, skewed");
     check_sddmm(uniform(1024, 1024, 128, 128, 20, 12), 64, cus, "sddmm 128x128 blocks");
     check_sddmm(banded(8192, 32, 8, 655, 20), 128, cus, "sddmm banded 8192^2 (column bands)");
+    for (int64_t N : {128, 160, 224, 288, 384, 480, 640, 896, 1056, 1152, 1536, 2176})
+        check_spmm_stream_ragged(uniform(4096, 4096, 32, 32, 4096, 1), N, cus, false,
+                                 "stream 25% N=" + std::to_string(N));
+    check_spmm_stream_ragged(skewed(2048, 2048, 64, 32, 300, 41), 416, cus, false, "stream 64x32, duplicates N=416");
+    check_spmm_stream_ragged(uniform(4096, 4096, 32, 32, 2000, 42), 1184, cus, true, "stream pairs N=1184");
+    check_spmm_stream_ragged(uniform(1024, 1024, 32, 32, 0, 9), 160, cus, false, "stream empty N=160");
     check_sddmm_tiles(uniform(4096, 4096, 32, 32, 4096, 21), 512, cus, {32, 128, 2}, "sddmm tiles 32x32 25%");
     check_sddmm_tiles(skewed(2048, 1920, 64, 96, 200, 22), 512, cus, {64, 128, 2}, "sddmm tiles 64x96, skewed");
     check_sddmm_tiles(uniform(2048, 2048, 128, 64, 100, 23), 512, 16, {32, 128, 4}, "sddmm tiles 128x64 in 32 rows");

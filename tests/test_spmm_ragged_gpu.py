@@ -1,0 +1,64 @@
+"""SpMM with N that is no multiple of 128 on the GPU against the oracle: the
+persistent kernel's overlapping last tile (N >= 128), for single stripes,
+stripe pairs and the skewed-row variant, in C whose rows are wider than N.
+
+Bound: both sides add the same n products (exact in fp32) of values in [-1, 1]
+in fp32 in different orders: each is off by at most n^2 * 2^-24; twice that is
+allowed, and one bf16 rounding (2^-8) on bf16 output."""
+import numpy as np
+import pytest
+
+from helpers import W, bsr_of, capi, golden_spmm, spmm_k_eff, strided_run, with_values
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(a, N, out_dtype, persistent, pad=32):
+    b = W.dense_content(a.W, N, "RAND", np.random.default_rng(N))
+    plan = capi.SpmmPlan(bsr_of(a), N, out_dtype)
+    assert (plan.info()["persistent"] == 1) == persistent, plan.info()
+    import torch
+    got, after, before = strided_run(
+        a, b, out_dtype, N, N + pad,
+        lambda da, bw, cw: plan.run(da, bw, cw, stream=torch.cuda.current_stream().cuda_stream))
+    plan.close()
+    np.testing.assert_array_equal(after.view(np.uint8), before.view(np.uint8), err_msg="C's padding was written")
+    gold = golden_spmm(a, b)
+    n = spmm_k_eff(a).astype(np.float64)
+    bound = 2 * (n * n + 1) * 2.0 ** -24 + (2.0 ** -8 * np.abs(gold) if out_dtype == "bf16" else 0)
+    err = np.abs(got.astype(np.float64) - gold)
+    assert np.isfinite(got).all() and np.all(err <= bound), (N, out_dtype, err.max())
+
+
+def _matrix(H, Wd, R, C, density, seed):
+    rng = np.random.default_rng(seed)
+    n = max(1, round(density * (H // R) * (Wd // C)))
+    return with_values(W.random_positions(H, Wd, R, C, n, rng), "RAND", seed=seed)
+
+
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N", [128, 160, 224, 256, 288, 480, 1184])
+def test_persistent_partial_tiles(N, out_dtype):
+    print(N, out_dtype, flush=True)
+    _check(_matrix(1056, 1120, 32, 32, 0.15, 1), N, out_dtype, True)
+    _check(_matrix(1024, 4032, 32, 96, 0.1, 2) if N < 1000 else _matrix(4096, 2048, 32, 32, 0.01, 3), N, out_dtype, True)
+
+
+@pytest.mark.parametrize("variant", ["128,14,16,4,1,2,1", "128,8,8,2,1,2,2", "128,6,12,2,1,1,1"])
+def test_variants_partial_tiles(variant, monkeypatch):
+    monkeypatch.setenv("BSP_SPMM_STREAM_VARIANT", variant)
+    monkeypatch.setenv("BSP_SPMM_PAIRS", "2" if variant.endswith(",2") else "0")
+    for N in (160, 416):
+        print(variant, N, flush=True)
+        _check(_matrix(2080, 1024, 32, 32, 0.2, 4), N, "f32", True)
+
+
+def test_no_alloc_still_refuses():
+    import torch
+    a = _matrix(256, 256, 32, 32, 0.3, 5)
+    t = torch.zeros(1 << 16, dtype=torch.int16, device="cuda")
+    d = bsr_of(a).desc()
+    import ctypes
+    st = capi.load().bsp_spmm_noalloc(ctypes.byref(d), t.data_ptr(), t.data_ptr(), 160, 160, t.data_ptr(), 160,
+                                      capi.DTYPE_BF16, 0, None)
+    assert st == capi.BSP_ERR_UNSUPPORTED
