@@ -42,6 +42,7 @@ struct bsp_plan {
     int32_t sddmm_one_shot = 0;  // SDDMM: the one-shot kernel runs this plan
     int32_t tile = 0;            // SDDMM, SpGEMM: the tile kernel runs this plan on tiles of that height
     bsp::SddmmTileVariant sddmm_tile{};
+    int32_t narrow = 0;          // SpMM of fewer than 128 columns: waves of spmm_narrow_kernel
     int32_t cb_shift = 0;        // SDDMM tiles: log2 of the column chunks' width
     // SpMM persistent kernel: variant, unit records and A words (the B words
     // go in d_ent_off, the workgroup heads in d_wgs; d_apw with stripe pairs).
@@ -605,6 +606,16 @@ int make_spmm_plan(bsp_plan** out, int kind, const bsp_bsr_desc* a, int64_t N, i
     p->C = a->C;
     p->nblocks = a->nblocks;
     fill_info_spmm(s, &p->info);
+    if (kind == 1 && N < 128 && s.group == 1 && s.tile_n == 128) {
+        // Eight waves while the items fit the compute units once (and at N =
+        // 32, where two such workgroups fit one); else four, whose LDS lets
+        // two or three share a compute unit: 16384 x 4096, 5%, N = 64 / 96: 6.7
+        // / 8.6 us with eight, 5.0 / 6.5 with four.  N = 96 with many short
+        // items stays with the per-item kernel (6.0 there).
+        const int64_t items = p->info.n_items, entries = p->info.n_entries;
+        p->narrow = N == 32 || items <= cus ? 8 : N == 96 && entries < 8 * items ? 0 : 4;
+        if (p->narrow) p->info.waves = p->narrow;
+    }
     if (kind == 3) {
         p->info.kind = 3;
         p->info.stages = bsp::kAttentionStages;
@@ -716,7 +727,7 @@ int bsp_spmm(const bsp_plan* p, const uint16_t* a_vals, const uint16_t* b, int64
         e = bsp::launch_spmm_stream(sa, p->stream_variant, p->out_dtype == BSP_DTYPE_BF16, p->info.grid,
                                     (hipStream_t)stream);
     } else {
-        const bsp::SpmmVariant v{p->info.tile_n, p->info.stages, p->info.group, p->info.waves};
+        const bsp::SpmmVariant v{p->info.tile_n, p->info.stages, p->info.group, p->info.waves, p->narrow};
         e = bsp::launch_spmm(args, v, p->out_dtype == BSP_DTYPE_BF16, p->info.grid, p->info.n_split_rows,
                              (hipStream_t)stream);
     }

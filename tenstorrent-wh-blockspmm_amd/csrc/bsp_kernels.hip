@@ -558,6 +558,139 @@ __global__ __launch_bounds__(256) void spmm_kernel(SpmmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+// SpMM with fewer than 128 columns (N = 32 NT: a decode batch).  A workgroup
+// takes the same work items and the one tile of the kernel above, whose four
+// waves of 32 columns would mostly multiply columns past N; here its NW waves
+// split the item's entries (wave w takes entries w, w + NW, ...), each through
+// a two-stage ring of its own (2 KB of A, 2 KB x NT of B), and the partial
+// tiles are added in LDS in wave order.  What is left is the latency of one
+// round of loads: up to 2 NW entries of an item are in flight at once, and no
+// wave waits for another before the sum.  us of the kernel above : this one,
+// N = 32 / 64 / 96: 4128 x 3104, 8% 5.2 : 3.0 / 5.2 : 3.7 / 5.2 : 4.5; 4096^2
+// 25% 10.2 : 4.6 / 10.3 : 6.2 / 10.4 : 7.9; 2048 x 16384, 40% 39.6 : 12.2 /
+// 40.0 : 17.5 / 40.4 : 22.2; 16384^2 10% 17.9 : 12.0 / 19.2 : 15.1 / 20.3 :
+// 18.5 (four waves at N = 64 and 96).
+template <int NT, int NW, bool OUT_BF16>
+__global__ __launch_bounds__(64 * NW) void spmm_narrow_kernel(SpmmArgs p) {
+    using namespace spmm_detail;
+    constexpr int ROW = 64 * NT;              // bytes of a row of the B slice
+    constexpr int STAGE = kA_BYTES + 32 * ROW;
+    constexpr int BL = 2 * NT;                // 1 KB loads of B per entry
+    constexpr int PER = 2 + BL;
+    static_assert(2 * STAGE >= NT * 4096, "a wave's partial tile fits its ring");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[NW * 2 * STAGE];
+    const SpmmWg it = load_const(p.wgs + blockIdx.x);
+    if (it.row < 0) return;  // idle slot (uniform)
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int l32 = lane & 31, q = lane >> 5;
+    const int n_item = it.e_end - it.e_begin;
+    const int n = n_item > wave ? (n_item - wave + NW - 1) / NW : 0;  // this wave's entries
+    uint8_t* ring = smem + wave * 2 * STAGE;
+    const uint32_t lds = lds_address(ring);
+
+    // Words of the wave's entries 64c .. 64c+63 in lanes.
+    const int64_t* ents = p.ents + it.e_begin + wave;
+    uint32_t lo = 0, hi = 0;
+    auto fetch = [&](int base) {
+        if (base + lane < n) {
+            const int64_t w = ents[(int64_t)(base + lane) * NW];
+            lo = (uint32_t)w;
+            hi = (uint32_t)((uint64_t)w >> 32);
+        }
+        __asm__ volatile("" : "+v"(lo), "+v"(hi));
+    };
+    // B slice: row k at k * ROW, its 16-byte chunk c at slot c ^ swz(k): at 128
+    // bytes a row, rows k and k+2 share banks.
+    auto swz = [](int k) { return NT == 2 ? 4 * ((k >> 1) & 1) : 0; };
+    uint32_t a_voff[2], b_voff[BL];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) a_voff[j] = 2 * a_row_load_offset(j, lane, p.lda);
+#pragma unroll
+    for (int j = 0; j < BL; ++j) {
+        const int slot = j * 64 + lane, k = slot / (4 * NT), c = (slot % (4 * NT)) ^ swz(k);
+        b_voff[j] = (uint32_t)(2 * ((int64_t)k * p.ldb + 8 * c));
+    }
+    auto issue = [&](int e, int stage) {
+        if ((e & 63) == 0) fetch(e);
+        const uint16_t* a = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, e & 63) * 32;
+        const uint16_t* b = p.b + (int64_t)(uint32_t)__builtin_amdgcn_readlane(lo, e & 63) * p.ldb;
+        const uint32_t at = lds + stage * STAGE;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) gl_lds16_s(a_voff[j], a, at + j * 1024);
+#pragma unroll
+        for (int j = 0; j < BL; ++j) gl_lds16_s(b_voff[j], b, at + kA_BYTES + j * 1024);
+    };
+    int b_rd[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int k = 8 * q + ((lane & 15) >> 2), col = 32 * nt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+        b_rd[nt] = kA_BYTES + k * ROW + 16 * ((col >> 3) ^ swz(k)) + 2 * (col & 7);  // + 16 ROW per k-step, 4 ROW per half
+    }
+    f32x16 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[nt][v] = 0.0f;
+    if (n > 0) issue(0, 0);
+    if (n > 1) issue(1, 1);
+    for (int e = 0; e < n; ++e) {
+        if (e + 1 < n)
+            wait_vmcnt<PER>();
+        else
+            wait_vmcnt<0>();
+        const uint8_t* st = ring + (e & 1) * STAGE;
+        u32x4 a[2], b[2][NT];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            a[s] = *(const u32x4*)(st + a_row_read_offset(l32, q, s));
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const u32x4 x = ld_tr_b16(st + b_rd[nt] + s * 16 * ROW), y = ld_tr_b16(st + b_rd[nt] + (s * 16 + 4) * ROW);
+                b[s][nt] = u32x4{x.x, x.y, y.x, y.y};
+            }
+        }
+        wait_lgkm0();
+        if (e + 2 < n) issue(e + 2, e & 1);
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma32(a[s], b[s][nt], acc[nt]);
+    }
+    // The partial tiles meet in LDS (each in its wave's ring, whose loads have
+    // all been consumed): value (nt, v) of lane l at ((nt * 16 + v) * 64 + l).
+    // (The products may still be in the matrix core here, behind a branch.)
+    __asm__ volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        __asm__ volatile("" : "+v"(acc[nt]));
+#pragma unroll
+        for (int v = 0; v < 16; ++v) ((float*)ring)[(nt * 16 + v) * 64 + lane] = acc[nt][v];
+    }
+    wait_lgkm0();
+    barrier_no_fence();
+    float* piece = it.slot >= 0 ? p.ws + ((int64_t)it.slot * p.n_tiles + it.tile) * (16 * 256) : nullptr;
+#pragma unroll
+    for (int i = 0; i < 16 * NT / NW; ++i) {
+        const int at = i * (64 * NW) + tid;
+        float sum = 0.0f;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += ((const float*)(smem + w * 2 * STAGE))[at];
+        const int nt = at >> 10, v = (at >> 6) & 15;
+        if (piece) {  // a piece of a split row: its partial tile, for spmm_reduce_kernel
+            piece[v * 256 + nt * 64 + lane] = sum;
+        } else {
+            const int64_t row = (int64_t)it.row * 32 + 8 * (v >> 2) + 4 * q + (v & 3);
+            const int64_t idx = row * p.ldc + 32 * nt + l32;
+            if (OUT_BF16)
+                store_out(&((uint16_t*)p.c)[idx], f32_to_bf16_rne(sum));
+            else
+                store_out(&((float*)p.c)[idx], sum);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
 // SpMM over row groups: a workgroup takes RW (2, 4 or 8) consecutive 32-row
 // stripes of one block row (R >= 64) and one 128-column tile, so each entry's
 // B panel is loaded once and multiplied by the RW stripes' A sub-blocks
@@ -2338,10 +2471,38 @@ __global__ __launch_bounds__(256) void spgemm_kernel(SpgemmArgs p) {
 }
 
 // ---------------------------------------------------------------------------
+template <int NT, int NW>
+static void launch_spmm_narrow_t(const SpmmArgs& a, bool out_bf16, int grid, hipStream_t stream) {
+    if (out_bf16)
+        hipLaunchKernelGGL((spmm_narrow_kernel<NT, NW, true>), dim3(grid), dim3(64 * NW), 0, stream, a);
+    else
+        hipLaunchKernelGGL((spmm_narrow_kernel<NT, NW, false>), dim3(grid), dim3(64 * NW), 0, stream, a);
+}
+
+static void launch_spmm_narrow(const SpmmArgs& a, int waves, bool out_bf16, int grid, hipStream_t stream) {
+    switch (a.N / 32) {
+        case 1: launch_spmm_narrow_t<1, 8>(a, out_bf16, grid, stream); break;
+        case 2:
+            if (waves == 8)
+                launch_spmm_narrow_t<2, 8>(a, out_bf16, grid, stream);
+            else
+                launch_spmm_narrow_t<2, 4>(a, out_bf16, grid, stream);
+            break;
+        default:
+            if (waves == 8)
+                launch_spmm_narrow_t<3, 8>(a, out_bf16, grid, stream);
+            else
+                launch_spmm_narrow_t<3, 4>(a, out_bf16, grid, stream);
+    }
+}
+
 template <int NTW, int S, int G>
-static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_split, int waves, hipStream_t stream) {
+static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_split, int waves, int narrow,
+                          hipStream_t stream) {
     if constexpr (G == 1) {
-        if (out_bf16)
+        if (narrow)
+            launch_spmm_narrow(a, narrow, out_bf16, grid, stream);
+        else if (out_bf16)
             hipLaunchKernelGGL((spmm_kernel<NTW, S, true>), dim3(grid), dim3(256), 0, stream, a);
         else
             hipLaunchKernelGGL((spmm_kernel<NTW, S, false>), dim3(grid), dim3(256), 0, stream, a);
@@ -2393,10 +2554,11 @@ static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_spli
 hipError_t launch_spmm(const SpmmArgs& a, const SpmmVariant& v, bool out_bf16, int grid, int n_split,
                        hipStream_t stream) {
     if (grid <= 0) return hipSuccess;
-    if (!spmm_variant_supported(v)) return hipErrorInvalidValue;
+    if (!spmm_variant_supported(v) || (v.narrow && (v.tile_n != 128 || v.group != 1 || a.N >= 128)))
+        return hipErrorInvalidValue;
 #define BSP_SPMM_CASE(TN, S, G)                                                   \
     if (v.tile_n == TN && v.stages == S && v.group == G) {                       \
-        launch_spmm_t<TN / 128, S, G>(a, out_bf16, grid, n_split, v.waves, stream); \
+        launch_spmm_t<TN / 128, S, G>(a, out_bf16, grid, n_split, v.waves, v.narrow, stream); \
         return hipGetLastError();                                                \
     }
     BSP_SPMM_VARIANTS(BSP_SPMM_CASE)

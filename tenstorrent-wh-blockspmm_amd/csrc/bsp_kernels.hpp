@@ -261,7 +261,8 @@ struct SpmmVariant {
     int tile_n;
     int stages;
     int group;
-    int waves = 4;  // 256-column row groups: 8 (default) or 4 waves per workgroup
+    int waves = 4;   // 256-column row groups: 8 (default) or 4 waves per workgroup
+    int narrow = 0;  // N < 128, single stripes: spmm_narrow_kernel with that many waves (4 or 8; 0: spmm_kernel)
 };
 
 inline bool spmm_variant_supported(const SpmmVariant& v) {

@@ -62,3 +62,17 @@ def test_no_alloc_still_refuses():
     st = capi.load().bsp_spmm_noalloc(ctypes.byref(d), t.data_ptr(), t.data_ptr(), 160, 160, t.data_ptr(), 160,
                                       capi.DTYPE_BF16, 0, None)
     assert st == capi.BSP_ERR_UNSUPPORTED
+
+
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("N", [32, 64, 96])
+def test_narrow(N, out_dtype, monkeypatch):
+    """Fewer than 128 columns: items of no, one, few and (past the 64 words a
+    wave holds: more than 512) many entries, larger blocks, split rows."""
+    print(N, out_dtype, flush=True)
+    _check(_matrix(1056, 1120, 32, 32, 0.02, 1), N, out_dtype, False)
+    _check(_matrix(512, 4032, 64, 96, 0.3, 2), N, out_dtype, False)
+    full = W.fill_row(64, 32 * 700, 32, 32, 1 + 700)  # a full row and a row of one block
+    _check(with_values(full, "RAND", seed=3), N, out_dtype, False)
+    monkeypatch.setenv("BSP_SPMM_SPLIT", "9")
+    _check(_matrix(256, 2048, 32, 32, 0.5, 4), N, out_dtype, False)
