@@ -618,7 +618,8 @@ int make_spmm_plan(bsp_plan** out, int kind, const bsp_bsr_desc* a, int64_t N, i
     }
     if (kind == 3) {
         p->info.kind = 3;
-        p->info.stages = bsp::kAttentionStages;
+        p->info.stages = 1;
+        p->info.waves = bsp::attention_waves(N, p->info.n_items, cus);
     }
     hipError_t e = upload((bsp::SpmmWg**)&p->d_wgs, bsp::spmm_wg_records(s));
     if (e == hipSuccess) e = upload(&p->d_ent_off, bsp::spmm_packed_entries(s));
@@ -772,7 +773,7 @@ int bsp_attention(const bsp_plan* p, const uint16_t* mask_vals, const uint16_t* 
     args.k = k;
     args.ldq = ldq;
     args.ldk = ldk;
-    hipError_t e = bsp::launch_attention(args, (int)d, p->out_dtype == BSP_DTYPE_BF16, p->info.grid,
+    hipError_t e = bsp::launch_attention(args, (int)d, p->info.waves, p->out_dtype == BSP_DTYPE_BF16, p->info.grid,
                                          p->info.n_split_rows, (hipStream_t)stream);
     if (e != hipSuccess) return hip_fail(e, "attention launch");
     return BSP_OK;

@@ -192,14 +192,8 @@ namespace spmm_detail {
 // With OVERLAP = false (one operand set, for kernels whose accumulators leave
 // no registers for a second) entry k is multiplied before the barrier and
 // entry k+1's reads follow it.  landed() runs once entry 0 (and every load
-// issued before it) has landed and is visible to all waves.  With MIX (and
-// OVERLAP), entry k+1's reads and entry k's products form one scheduling
-// region.  With XCHG (and OVERLAP), read() may leave LDS data that the other
-// waves' multiply() of the same entry reads: a barrier then also follows
-// landed() (whose LDS reads complete first) and precedes a multiply() that no
-// ring step separates from its entry's read().
-template <int S, int PER, bool OVERLAP, class Ops, bool MIX = false, bool XCHG = false, class Issue, class Read,
-          class Multiply, class Landed>
+// issued before it) has landed and is visible to all waves.
+template <int S, int PER, bool OVERLAP, class Ops, class Issue, class Read, class Multiply, class Landed>
 __device__ __forceinline__ void run_ring(int n, Issue&& issue, Read&& read, Multiply&& multiply,
                                          Landed&& landed) {
     static_assert(PER * (S - 2) < 64, "vmcnt budget");
@@ -211,13 +205,6 @@ __device__ __forceinline__ void run_ring(int n, Issue&& issue, Read&& read, Mult
     wait_stages<PER, S - 2>(n - 1);  // entry 0 landed
     barrier_no_fence();
     landed();
-    auto xchg = [] {
-        if constexpr (XCHG) {
-            spmm_detail::wait_lgkm0();
-            barrier_no_fence();
-        }
-    };
-    xchg();
     if (S - 1 < n) issue(S - 1, S - 1);
     read(0, o0);
     int stage = 0;  // stage of entry k
@@ -249,43 +236,38 @@ __device__ __forceinline__ void run_ring(int n, Issue&& issue, Read&& read, Mult
     // do not depend on; the reads must be in flight while the MFMAs run.
     auto fence_sched = [] { __builtin_amdgcn_sched_barrier(0); };
     if constexpr (OVERLAP) {
-        auto fence_rm = [&] {
-            if constexpr (!MIX) fence_sched();
-        };
         Ops o1;
         for (; k + S + 1 < n; k += 2) {
             sync_full(k);
             read(stage, o1);
-            fence_rm();
+            fence_sched();
             multiply(o0);
             fence_sched();
             sync_full(k + 1);
             read(stage, o0);
-            fence_rm();
+            fence_sched();
             multiply(o1);
             fence_sched();
         }
         for (; k + 2 < n; k += 2) {
             sync(k);
             read(stage, o1);
-            fence_rm();
+            fence_sched();
             multiply(o0);
             fence_sched();
             sync(k + 1);
             read(stage, o0);
-            fence_rm();
+            fence_sched();
             multiply(o1);
             fence_sched();
         }
         if (k + 1 < n) {
             sync(k);
             read(stage, o1);
-            fence_rm();
+            fence_sched();
             multiply(o0);
-            xchg();
             multiply(o1);
         } else {
-            xchg();
             multiply(o0);
         }
     } else {
@@ -439,14 +421,12 @@ struct BSlice {
 
 // B operands of NT 32-column tiles (from column col0 of a TN-wide slice) by
 // transpose reads.  The rows read for k-step s2, lane half q, 4-row group h
-// are 16*s2 + 8*q + 4*h (the MFMA's own order) or, with permuted, 16*s2 +
-// 8*h + 4*q (the order in which a 32x32 MFMA result holds its rows, for an A
-// operand built from a result).
+// are 16*s2 + 8*q + 4*h (the MFMA's own order).
 template <int TN, int NT>
 struct BReads {
     int rd[2][2][NT];  // LDS offsets [k-step][4-row group][tile]
 
-    __device__ __forceinline__ BReads(int lane, int col0, bool permuted) {
+    __device__ __forceinline__ BReads(int lane, int col0) {
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2)
 #pragma unroll
@@ -454,8 +434,7 @@ struct BReads {
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt) {
                     const int g = lane >> 4;
-                    const int r = 16 * s2 + (permuted ? 8 * h + 4 * (g >> 1) : 8 * (g >> 1) + 4 * h) +
-                                  ((lane & 15) >> 2);
+                    const int r = 16 * s2 + 8 * (g >> 1) + 4 * h + ((lane & 15) >> 2);
                     const int col = col0 + nt * 32 + 16 * (g & 1) + 4 * (lane & 3);
                     const int c = col >> 3;
                     rd[s2][h][nt] = r * (2 * TN) + 16 * (c ^ (4 * (r & 3))) + 2 * (col & 7);
@@ -512,7 +491,7 @@ __global__ __launch_bounds__(256) void spmm_kernel(SpmmArgs p) {
     const int l32 = lane & 31, q = lane >> 5;
     const uint32_t lds0 = lds_address(smem);
     const Slice bsl(wave, lane, it.tile * Slice::TN, p.N, p.ldb);
-    const BReads<Slice::TN, NTW> brd(lane, wave * NTW * 32, false);
+    const BReads<Slice::TN, NTW> brd(lane, wave * NTW * 32);
 
     // Loads of one entry, per wave: lanes 0-31 fetch A segment `wave` (lane
     // 8*j + i loads A[8*wave + i][8*j .. +7]) and the wave's pieces of the B slice.
@@ -725,7 +704,7 @@ __global__ __launch_bounds__(256, 2) void spmm_group_kernel(SpmmArgs p) {
     const int wr = wave / WC, wc = wave % WC;
     const uint32_t lds0 = lds_address(smem);
     const Slice bsl(wave, lane, it.tile * Slice::TN, p.N, p.ldb);
-    const BReads<Slice::TN, NT> brd(lane, wc * NT * 32, false);
+    const BReads<Slice::TN, NT> brd(lane, wc * NT * 32);
 
     // A of one entry: 4*RW segments of 512 bytes (sub-block L/4, rows
     // 8*(L%4) .. +7); segment L lands at L*512, and wave w's load j covers
@@ -852,7 +831,7 @@ __global__ __launch_bounds__(64 * NW, RW <= 4 && S == 3 ? 2 : 1) void spmm_group
     const int wr = wave / WC, wc = wave % WC;
     const uint32_t lds0 = lds_address(smem);
     const Slice bsl(wave, lane, it.tile * Slice::TN, p.N, p.ldb);
-    const BReads<Slice::TN, NT> brd(lane, wc * NT * 32, false);
+    const BReads<Slice::TN, NT> brd(lane, wc * NT * 32);
 
     // A without pairs: of one entry, 4*RW segments of 512 bytes (sub-block
     // L/4, rows 8*(L%4) .. +7); segment L lands at L*512, and wave w's load j
@@ -1277,7 +1256,7 @@ __global__ __launch_bounds__(64 * (4 * SR + 1 + NBW) * PIPES) void spmm_stream_k
     // with stripe pairs the second) and columns (w%4)*NTW*32 .. of its tile.
     const int l32 = lane & 31, q = lane >> 5;
     const int half = wave >> 2, wc = wave & 3;
-    const BReads<TN, NTW> brd(lane, wc * NTW * 32, false);
+    const BReads<TN, NTW> brd(lane, wc * NTW * 32);
     const int a_rd0 = a_row_read_offset(l32, q, 0) + half * kA_BYTES;
     const int a_rd1 = a_row_read_offset(l32, q, 1) + half * kA_BYTES;
     f32x16 acc[NTW];
@@ -1556,7 +1535,7 @@ __global__ __launch_bounds__(64 * (8 + 1 + NBW), 1) void spmm_sweep_kernel(SpmmS
     // ---- MFMA waves.
     const int l32 = lane & 31, q = lane >> 5;
     const int group = wave >> 2, wc = wave & 3;
-    const BReads<TN, 1> brd(lane, wc * 32, false);
+    const BReads<TN, 1> brd(lane, wc * 32);
     const int a_rd0 = a_row_read_offset(l32, q, 0);
     const int a_rd1 = a_row_read_offset(l32, q, 1);
     // (The lambdas are forced inline: one left out of line would take acc by
@@ -1742,138 +1721,222 @@ __global__ __launch_bounds__(64 * (8 + 1 + NBW), 1) void spmm_sweep_kernel(SpmmS
 
 // ---------------------------------------------------------------------------
 // Block-sparse attention pair, fused: O = S * V with S = bf16(mask (.) (Q*K^T))
-// at the mask's blocks, S never leaving the compute unit.  Same schedule and
-// ring as the SpMM (the mask plays A, V plays B, one 128-column tile); each
-// ring stage also carries the entry's 32 x DK block of K.  Each wave computes
-// one 16 x 16 quadrant of the entry's S^T = K_blk * Q^T from LDS (its 16
-// queries of Q^T stay in registers), applies the mask, rounds to bf16 and
-// writes the quadrant to an S buffer in LDS; after the next ring barrier
-// every wave reads the whole 32 x 32 S from there as the A operand of
-// O += S * V.  Numerically the same as bsp_sddmm (column-major Y = K, bf16
-// output) followed by bsp_spmm with the same structure, up to the fp32
-// summation order of Q K^T.
-template <int DK, int S, bool OUT_BF16>
-__global__ __launch_bounds__(256) void attention_kernel(AttentionArgs pa) {
+// at the mask's blocks, S never leaving the compute unit.  Same schedule as the
+// SpMM (the mask plays A, V plays B, one tile of all DK columns).  Numerically
+// the same as bsp_sddmm (column-major Y = K, bf16 output) followed by bsp_spmm
+// with the same structure, up to the order of the fp32 sums.
+//
+// The NW waves of a workgroup split an item's entries (wave w takes entries w,
+// w + NW, ...), each through a one-stage ring of its own, and add their partial
+// tiles in LDS in wave order.  A wave computes the whole S^T = K_blk * Q^T of
+// its entry from LDS and Q^T in registers; the 32x32 result holds, per lane,
+// one query's keys in the order 8 (v / 4) + 4 (lane / 32) + v % 4, so masked
+// and rounded it is the A operand of O += S * V as it stands, with V's rows
+// read in that order: no exchange between waves, and no barrier but the one
+// that publishes Q and the one before the sum.  K's part of the stage is
+// refilled once K is in registers, ahead of the products; mask and V once they
+// are.
+//
+// A stripe has 3 to some 30 entries, so a launch is the latency of its loads
+// and of its longest stripe: all four waves sharing each entry's products, one
+// entry after the other, took ~0.4 us an entry.  us a call there : here
+// (graph of 8 heads, bf16 O): 8 diagonals + 1% global blocks of 32, seq 8192, d
+// = 32 / 64 / 128 9.1 : 4.7 / 9.0 : 5.8 / 9.9 : 8.2; seq 1024 6.7 : 3.9 / 6.3 :
+// 4.3 / 6.9 : 5.8; 16 diagonals + 3%, seq 16384 18.2 : 12.8 / 20.2 : 13.9 /
+// 26.9 : 21.6; 16 + 5% of 128 x 128 blocks, seq 16384 45.3 : 23.7 / 50.8 : 26.6
+// / 69.8 : 42.6.  At d = 128 what is left is moving the operands: 18 KB an
+// entry, every XCD reading the K and V rows that its stripes' global blocks
+// name (two-stage rings, twice as much in flight, are slower there: 9.6 us at
+// seq 8192, 27.7 at 16384 with 16 diagonals).
+template <int DK, int NW, bool OUT_BF16>
+__global__ __launch_bounds__(64 * NW) void attention_kernel(AttentionArgs pa) {
     using namespace spmm_detail;
-    using Slice = BSlice<1>;
     const SpmmArgs& p = pa.s;
-    constexpr int K_BYTES = 64 * DK;              // 32 keys x DK bf16
-    constexpr int K_LANES = DK >= 64 ? 64 : 32;    // lanes per K load instruction
-    constexpr int KI = K_BYTES / 4 / (16 * K_LANES);  // K load instructions per wave
-    constexpr int PER = 1 + KI + Slice::BI;
-    constexpr int K_RING = S * kA_BYTES;
-    constexpr int B_RING = K_RING + S * K_BYTES;
-    constexpr int Q_AREA = B_RING + S * Slice::BYTES;
-    static_assert(KI >= 1 && DK % 32 == 0 && DK <= 128, "head dimension");
-    // The Q area holds Q, then (Q in registers) the two 2 KB S buffers.
-    __shared__ __attribute__((aligned(1024))) uint8_t smem[Q_AREA + (K_BYTES > 4096 ? K_BYTES : 4096)];
+    constexpr int NT = DK / 32;                 // 32-column tiles of O
+    constexpr int ROW = 2 * DK;                 // bytes of a Q, K or V row
+    constexpr int CPR = DK / 8;                 // its 16-byte chunks
+    constexpr int BLOCK = 32 * ROW;             // a 32-row block of Q, K or V
+    constexpr int LB = BLOCK / 1024;            // 1 KB loads of one
+    constexpr int K_AT = kA_BYTES, V_AT = K_AT + BLOCK, STAGE = V_AT + BLOCK;
+    constexpr int Q_AT = NW * STAGE;
+    static_assert(DK == 32 || DK == 64 || DK == 128, "head dimension");
+    static_assert(STAGE >= NT * 4096, "a wave's partial tile fits its stage");
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[Q_AT + BLOCK];
 
     const SpmmWg it = load_const(p.wgs + blockIdx.x);
-    if (it.row < 0) return;
-    const int tid = threadIdx.x;
-    const int lane = tid & 63;
+    if (it.row < 0) return;  // idle slot (uniform)
+    const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int l32 = lane & 31, q = lane >> 5;
-    const uint32_t lds0 = lds_address(smem);
-    const Slice bsl(wave, lane, 0, p.N, p.ldb);
-    const BReads<Slice::TN, 1> brd(lane, wave * 32, false);
+    const int n_item = it.e_end - it.e_begin;
+    const int n = n_item > wave ? (n_item - wave + NW - 1) / NW : 0;  // this wave's entries
+    const uint8_t* st = smem + wave * STAGE;
+    const uint32_t lds0 = lds_address(smem), lds = lds0 + wave * STAGE;
 
-    // K blocks and the stripe's Q rows in LDS as 16-byte chunks (c, row r) at
-    // (32c + r) * 16, so that the operand of step s of row l32 (chunk 2s + q)
-    // is one conflict-free ds_read_b128.  Wave w loads chunks [w*DK, (w+1)*DK).
-    uint32_t k_voff[KI];  // byte offsets from the block's first key row
-    int64_t q_goff[KI];
+    // Q and K blocks: row r at r * ROW, its chunk c at slot c ^ qk_swz(r), so
+    // that the 16 rows of which a quarter of a wave reads one chunk cover the
+    // 64 banks.  V: chunk c of row k at slot c ^ v_swz(k), for transpose reads.
+    auto qk_swz = [](int r) { return (r / (16 / CPR)) % CPR; };
+    auto v_swz = [](int k) { return DK == 128 ? 4 * (k & 3) : DK == 64 ? 4 * ((k >> 1) & 1) : 0; };
+    if (n_item > 0)
+        for (int j = wave; j < LB; j += NW) {
+            const int r = (j * 64 + lane) / CPR, c = lane % CPR ^ qk_swz(r);
+            gl_lds16(pa.q + ((int64_t)it.row * 32 + r) * pa.ldq + 8 * c, lds0 + Q_AT + j * 1024);
+        }
+
+    // Words of the wave's entries 64c .. 64c+63 in lanes.
+    const int64_t* ents = p.ents + it.e_begin + wave;
+    uint32_t lo = 0, hi = 0;
+    auto fetch = [&](int base) {
+        if (base + lane < n) {
+            const int64_t w = ents[(int64_t)(base + lane) * NW];
+            lo = (uint32_t)w;
+            hi = (uint32_t)((uint64_t)w >> 32);
+        }
+        __asm__ volatile("" : "+v"(lo), "+v"(hi));
+    };
+    uint32_t m_voff[2], k_voff[LB], v_voff[LB];  // byte offsets (ldk, ldv < 2^26: 32 rows span less than 4 GB)
 #pragma unroll
-    for (int j = 0; j < KI; ++j) {
-        const int ci = wave * DK + j * K_LANES + (lane & (K_LANES - 1));
-        k_voff[j] = (uint32_t)(2 * ((int64_t)(ci & 31) * pa.ldk + 8 * (ci >> 5)));
-        q_goff[j] = (int64_t)(ci & 31) * pa.ldq + 8 * (ci >> 5);
+    for (int j = 0; j < 2; ++j) m_voff[j] = 2 * a_row_load_offset(j, lane, p.lda);
+#pragma unroll
+    for (int j = 0; j < LB; ++j) {
+        const int r = (j * 64 + lane) / CPR, c = lane % CPR;
+        k_voff[j] = (uint32_t)(2 * ((int64_t)r * pa.ldk + 8 * (c ^ qk_swz(r))));
+        v_voff[j] = (uint32_t)(2 * ((int64_t)r * p.ldb + 8 * (c ^ v_swz(r))));
     }
-    const int n = it.e_end - it.e_begin;
-    // Q of the stripe goes through the same DMA path ahead of the ring, so it
-    // has landed once entry 0 has; its operands are then read from LDS (plain
-    // global loads here would be waited for inside the loop by the compiler,
-    // which cannot see that they completed, draining the ring every entry).
+    uint32_t key = 0;  // first key of the block whose loads were issued last
+    auto issue_k = [&](int e) {
+        if ((e & 63) == 0) fetch(e);
+        key = __builtin_amdgcn_readlane(lo, e & 63);
+        const uint16_t* kb = pa.k + (int64_t)key * pa.ldk;
+#pragma unroll
+        for (int j = 0; j < LB; ++j) gl_lds16_s(k_voff[j], kb, lds + K_AT + j * 1024);
+    };
+    auto issue_mv = [&](int e) {
+        const uint16_t* m = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, e & 63) * 32;
+        const uint16_t* vb = p.b + (int64_t)key * p.ldb;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) gl_lds16_s(m_voff[j], m, lds + j * 1024);
+#pragma unroll
+        for (int j = 0; j < LB; ++j) gl_lds16_s(v_voff[j], vb, lds + V_AT + j * 1024);
+    };
+    int v_rd[NT];  // + 16 ROW per k-step, + 8 ROW per half: neither changes v_swz
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        const int k = 4 * q + ((lane & 15) >> 2), col = 32 * nt + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+        v_rd[nt] = V_AT + k * ROW + 16 * ((col >> 3) ^ v_swz(k)) + 2 * (col & 7);
+    }
+    f32x16 acc[NT];
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[nt][v] = 0.0f;
+
     if (n > 0) {
-        const uint16_t* qrow = pa.q + (int64_t)it.row * 32 * pa.ldq;
-#pragma unroll
-        for (int j = 0; j < KI; ++j)
-            if (lane < K_LANES) gl_lds16(qrow + q_goff[j], lds0 + Q_AREA + wave * DK * 16 + j * K_LANES * 16);
+        issue_k(0);
+        issue_mv(0);
+        wait_vmcnt<2 + 2 * LB>();  // this wave's part of Q has landed
+    } else {
+        wait_vmcnt<0>();
     }
-    // S = mask (.) Q K^T of an entry is computed in four 16 x 16 quadrants,
-    // one per wave: wave w takes keys ka = 16*(w%2) .. +15 and queries
-    // qb = 16*(w/2) .. +15, S^T quadrant = K[ka..][:] * Q[qb..][:]^T in DK/32
-    // 16x16x32 products.  Lane l holds Q[qb + l%16][32t + 8*(l/16) .. +7]
-    // for each 32-deep step t (the B operand).
-    const int ka = 16 * (wave & 1), qb = 16 * (wave >> 1);
-    const int l16 = lane & 15, g4 = lane >> 4;
-    u32x4 qv[DK / 32];
-    const uint32_t a_voff = 2 * ((8 * wave + (lane & 7)) * p.lda + 8 * ((lane & 31) >> 3));
-    const uint32_t a_lds = lds0 + wave * 512;
-    const uint32_t k_lds = lds0 + K_RING + wave * DK * 16;
-    const uint32_t b_lds = lds0 + B_RING + wave * Slice::BI * 1024;
-    EntryWords words(p.ents + it.e_begin, n, lane);
-    auto issue = [&](int e, int stage) {
-        uint32_t bw, aw;  // first key of the block, mask block offset / 32
-        words.get(e, lane, bw, aw);
-        if (lane < 32) gl_lds16_s(a_voff, p.a + (int64_t)aw * 32, a_lds + stage * kA_BYTES);
-        const uint16_t* kblk = pa.k + (int64_t)bw * pa.ldk;
+    barrier_no_fence();
+    u32x4 qv[DK / 16];
 #pragma unroll
-        for (int j = 0; j < KI; ++j)
-            if (lane < K_LANES) gl_lds16_s(k_voff[j], kblk, k_lds + stage * K_BYTES + j * K_LANES * 16);
-        bsl.issue(p.b, p.ldb, bw, b_lds + stage * Slice::BYTES);
-    };
-
-    // The quadrant's mask values of lane l: query qb + l%16, keys ka + 4*(l/16)
-    // .. +3, 8 bytes of the mask's row.  The mask is loaded without the SpMM A
-    // layout's chunk XOR: segment g, chunk j of row r at (8j + r%8) * 16.
-    const int mq = qb + l16, mkey = ka + 4 * g4;
-    const int m_rd = (mq >> 3) * 512 + (8 * (mkey >> 3) + (mq & 7)) * 16 + 2 * (mkey & 7);
-    // S of an entry in LDS (two buffers in the Q area, free once Q is in
-    // registers), bf16 row-major by query, 64 bytes a row, 16-byte chunk c of
-    // row r at position c ^ (r/4 % 4): each 16-lane quarter of the O
-    // operand read, and each half-wave of the quadrant write, covers every bank.
-    auto s_pos = [](int r, int key) { return r * 64 + 16 * ((key >> 3) ^ ((r >> 2) & 3)) + 2 * (key & 7); };
-    const int s_wr = s_pos(mq, mkey);
-    const int s_rd0 = s_pos(l32, 8 * q), s_rd1 = s_pos(l32, 16 + 8 * q);
-    f32x16 acc[1];
+    for (int t = 0; t < DK / 16; ++t)
+        qv[t] = *(const u32x4*)(smem + Q_AT + l32 * ROW + 16 * ((2 * t + q) ^ qk_swz(l32)));
+    for (int e = 0; e < n; ++e) {
+        wait_vmcnt<2 + LB>();  // K
+        u32x4 kv[DK / 16];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) acc[0][v] = 0.0f;
-
-    // Operands of one entry kept in registers: V's rows (its S is in LDS).
-    struct Operands {
-        u32x4 b[2][1];
-    };
-    int e_read = 0, e_mul = 0;  // entries read / multiplied so far (S buffer = entry % 2)
-    run_ring<S, PER, true, Operands, true, true>(
-        n, issue,
-        [&](int stage, Operands& o) {
-            const uint8_t* ks = smem + K_RING + stage * K_BYTES;
-            f32x4 sq = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int t = 0; t < DK / 16; ++t)
+            kv[t] = *(const u32x4*)(st + K_AT + l32 * ROW + 16 * ((2 * t + q) ^ qk_swz(l32)));
+        wait_lgkm0();
+        if (e + 1 < n) issue_k(e + 1);
+        f32x16 sc;  // S^T: keys x queries
 #pragma unroll
-            for (int t = 0; t < DK / 32; ++t)
-                sq = mfma16(*(const u32x4*)(ks + (32 * (4 * t + g4) + ka + l16) * 16), qv[t], sq);
-            const uint64_t mw = *(const uint64_t*)(smem + stage * kA_BYTES + m_rd);
-            const uint32_t m0 = (uint32_t)mw, m1 = (uint32_t)(mw >> 32);
-            // sq[v] = S^T[ka + 4*(l/16) + v][qb + l%16]: keys mkey + v of query mq.
-            const uint32_t lo = pack_bf16x2(sq[0] * __uint_as_float(m0 << 16), sq[1] * __uint_as_float(m0 & 0xffff0000u));
-            const uint32_t hi = pack_bf16x2(sq[2] * __uint_as_float(m1 << 16), sq[3] * __uint_as_float(m1 & 0xffff0000u));
-            *(uint64_t*)(smem + Q_AREA + (e_read & 1) * 2048 + s_wr) = (uint64_t)lo | ((uint64_t)hi << 32);
-            ++e_read;
-            brd.read(smem + B_RING + stage * Slice::BYTES, o.b);
-        },
-        [&](const Operands& o) {
-            const uint8_t* sx = smem + Q_AREA + (e_mul & 1) * 2048;
-            ++e_mul;
-            acc[0] = mfma32(*(const u32x4*)(sx + s_rd0), o.b[0][0], acc[0]);
-            acc[0] = mfma32(*(const u32x4*)(sx + s_rd1), o.b[1][0], acc[0]);
-        },
-        [&] {
+        for (int v = 0; v < 16; ++v) sc[v] = 0.0f;
 #pragma unroll
-            for (int t = 0; t < DK / 32; ++t)
-                qv[t] = *(const u32x4*)(smem + Q_AREA + (32 * (4 * t + g4) + qb + l16) * 16);
-        });
-    spmm_finish<1, OUT_BF16>(p, it, acc, tid);
+        for (int t = 0; t < DK / 16; ++t)
+            sc = mfma32(kv[t], qv[t], sc);
+        if (e + 1 < n)  // mask and V
+            wait_vmcnt<LB>();
+        else
+            wait_vmcnt<0>();
+        uint64_t mw[4];  // keys 8g + 4q .. +3 of query l32
+#pragma unroll
+        for (int g = 0; g < 4; ++g) mw[g] = *(const uint64_t*)(st + 64 * l32 + 16 * (g ^ ((l32 >> 2) & 3)) + 8 * q);
+        u32x4 b[2][NT];
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) {
+                const u32x4 x = ld_tr_b16(st + v_rd[nt] + s * 16 * ROW), y = ld_tr_b16(st + v_rd[nt] + (s * 16 + 8) * ROW);
+                b[s][nt] = u32x4{x.x, x.y, y.x, y.y};
+            }
+        wait_lgkm0();
+        if (e + 1 < n) issue_mv(e + 1);
+        u32x4 a[2];
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+            const uint32_t m0 = (uint32_t)mw[g], m1 = (uint32_t)(mw[g] >> 32);
+            a[g >> 1][2 * (g & 1)] =
+                pack_bf16x2(sc[4 * g] * __uint_as_float(m0 << 16), sc[4 * g + 1] * __uint_as_float(m0 & 0xffff0000u));
+            a[g >> 1][2 * (g & 1) + 1] =
+                pack_bf16x2(sc[4 * g + 2] * __uint_as_float(m1 << 16), sc[4 * g + 3] * __uint_as_float(m1 & 0xffff0000u));
+        }
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int nt = 0; nt < NT; ++nt) acc[nt] = mfma32(a[s], b[s][nt], acc[nt]);
+    }
+    // The partial tiles meet in LDS (each in its wave's stage, whose loads have
+    // all been consumed): value (nt, v) of lane l at ((nt * 16 + v) * 64 + l).
+    // (The products may still be in the matrix core here, behind a branch.)
+    __asm__ volatile("s_nop 15\n\ts_nop 7" ::: "memory");
+    float* part = (float*)(smem + wave * STAGE);
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt) {
+        __asm__ volatile("" : "+v"(acc[nt]));
+#pragma unroll
+        for (int v = 0; v < 16; ++v) part[(nt * 16 + v) * 64 + lane] = acc[nt][v];
+    }
+    wait_lgkm0();
+    barrier_no_fence();
+    // Four values of a row per thread; whole-row stores of 16 bytes (fp32) or 8
+    // where the output's alignment allows them.
+    const bool wide = ((uintptr_t)p.c % (OUT_BF16 ? 8 : 16)) == 0 && p.ldc % 4 == 0;
+    float* piece = it.slot >= 0 ? p.ws + ((int64_t)it.slot * p.n_tiles + it.tile) * (16 * 256) : nullptr;
+#pragma unroll
+    for (int i = tid; i < 8 * DK; i += 64 * NW) {
+        f32x4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int w = 0; w < NW; ++w) sum += ((const f32x4*)(smem + w * STAGE))[i];
+        const int nt = i >> 8, v = (i >> 4) & 15, l = 4 * (i & 15);  // of lanes l .. l+3
+        if (piece) {  // a piece of a split row: its partial tile, for spmm_reduce_kernel
+            *(f32x4*)(piece + v * 256 + nt * 64 + l) = sum;
+            continue;
+        }
+        const int64_t row = (int64_t)it.row * 32 + 8 * (v >> 2) + 4 * (l >> 5) + (v & 3);
+        const int64_t idx = row * p.ldc + 32 * nt + (l & 31);
+        if (OUT_BF16) {
+            uint16_t* o = (uint16_t*)p.c + idx;
+            const uint32_t s0 = pack_bf16x2(sum[0], sum[1]), s1 = pack_bf16x2(sum[2], sum[3]);
+            if (wide) {
+                store_out((uint64_t*)o, (uint64_t)s0 | ((uint64_t)s1 << 32));
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) store_out(o + x, (uint16_t)((x < 2 ? s0 : s1) >> (16 * (x & 1))));
+            }
+        } else {
+            float* o = (float*)p.c + idx;
+            if (wide) {
+                store_out((f32x4*)o, sum);
+            } else {
+#pragma unroll
+                for (int x = 0; x < 4; ++x) store_out(o + x, sum[x]);
+            }
+        }
+    }
 }
 
 // Adds the partials of each split row in piece order (deterministic) and
@@ -2597,12 +2660,21 @@ hipError_t launch_spmm_sweep(const SpmmSweepArgs& a, bool out_bf16, int grid, hi
     return hipGetLastError();
 }
 
-template <int DK>
-static void launch_attention_t(const AttentionArgs& a, bool out_bf16, int grid, int n_split, hipStream_t stream) {
+template <int DK, int NW>
+static void launch_attention_v(const AttentionArgs& a, bool out_bf16, int grid, hipStream_t stream) {
     if (out_bf16)
-        hipLaunchKernelGGL((attention_kernel<DK, kAttentionStages, true>), dim3(grid), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((attention_kernel<DK, NW, true>), dim3(grid), dim3(64 * NW), 0, stream, a);
     else
-        hipLaunchKernelGGL((attention_kernel<DK, kAttentionStages, false>), dim3(grid), dim3(256), 0, stream, a);
+        hipLaunchKernelGGL((attention_kernel<DK, NW, false>), dim3(grid), dim3(64 * NW), 0, stream, a);
+}
+
+template <int DK>
+static void launch_attention_t(const AttentionArgs& a, int waves, bool out_bf16, int grid, int n_split,
+                               hipStream_t stream) {
+    if (waves == 8)
+        launch_attention_v<DK, 8>(a, out_bf16, grid, stream);
+    else
+        launch_attention_v<DK, 4>(a, out_bf16, grid, stream);
     if (n_split > 0) {
         const int g = n_split * a.s.n_tiles;
         if (out_bf16)
@@ -2612,13 +2684,14 @@ static void launch_attention_t(const AttentionArgs& a, bool out_bf16, int grid, 
     }
 }
 
-hipError_t launch_attention(const AttentionArgs& a, int head_dim, bool out_bf16, int grid, int n_split,
+hipError_t launch_attention(const AttentionArgs& a, int head_dim, int waves, bool out_bf16, int grid, int n_split,
                             hipStream_t stream) {
     if (grid <= 0) return hipSuccess;
+    if (waves != 4 && waves != 8) return hipErrorInvalidValue;
     switch (head_dim) {
-        case 32: launch_attention_t<32>(a, out_bf16, grid, n_split, stream); break;
-        case 64: launch_attention_t<64>(a, out_bf16, grid, n_split, stream); break;
-        case 128: launch_attention_t<128>(a, out_bf16, grid, n_split, stream); break;
+        case 32: launch_attention_t<32>(a, waves, out_bf16, grid, n_split, stream); break;
+        case 64: launch_attention_t<64>(a, waves, out_bf16, grid, n_split, stream); break;
+        case 128: launch_attention_t<128>(a, waves, out_bf16, grid, n_split, stream); break;
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();

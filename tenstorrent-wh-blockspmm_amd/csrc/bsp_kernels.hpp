@@ -286,13 +286,18 @@ inline SpmmVariant spmm_default_variant(int tile_n, int group) {
 // Launches the SpMM kernel and, when the plan has split rows, the reduce kernel.
 hipError_t launch_spmm(const SpmmArgs& a, const SpmmVariant& v, bool out_bf16, int grid, int n_split,
                        hipStream_t stream);
-// Head dimensions of the fused attention kernel (one 128-column tile).
+// Head dimensions of the fused attention kernel (one tile).
 inline bool attention_head_dim_supported(int64_t d) { return d == 32 || d == 64 || d == 128; }
 constexpr int kAttentionTileN = 128;
-constexpr int kAttentionStages = 4;
+// Waves of its workgroups: eight while the items fit the compute units once,
+// and at d = 32, where three such workgroups fit one; else four, two workgroups
+// a compute unit (seq 16384, 16 diagonals + 3%, d = 64 / 128: 16.2 / 25.4 us
+// with eight, 13.9 / 21.6 with four; seq 8192, 8 + 1%, d = 64: 5.8 with eight,
+// 6.3 with four).
+inline int attention_waves(int64_t head_dim, int64_t items, int cus) { return head_dim == 32 || items <= cus ? 8 : 4; }
 
 // Launches the fused attention kernel and, for split rows, the reduce kernel.
-hipError_t launch_attention(const AttentionArgs& a, int head_dim, bool out_bf16, int grid, int n_split,
+hipError_t launch_attention(const AttentionArgs& a, int head_dim, int waves, bool out_bf16, int grid, int n_split,
                             hipStream_t stream);
 
 hipError_t launch_sddmm(const SddmmArgs& a, bool y_colmajor, bool out_bf16, int grid,

@@ -91,3 +91,55 @@ def test_fused_attention_empty_rows():
     for i, r in enumerate(rows):
         if not r:
             assert np.all(got[32 * i:32 * (i + 1)] == 0.0)
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("d", [32, 64, 128])
+def test_fused_attention_waves(d, out):
+    """Four and eight waves splitting an item's entries: items of one to nine
+    entries, more items than compute units, rows of more entries than a wave
+    holds words for (64 a wave), and rows of one entry."""
+    def check(mask, waves):
+        rng = np.random.default_rng(d)
+        std = np.float32(d ** -0.5)
+        q, k, v = (W.bf16_from_f32(rng.standard_normal((n, d), dtype=np.float32) * std)
+                   for n in (mask.H, mask.W, mask.W))
+        plan = capi.AttentionPlan(bsr_of(mask), d, out)
+        assert plan.info()["waves"] == waves, plan.info()
+        gold, s_arr = golden_attention(mask, q, k, v)
+        got = run_attention(mask, q, k, v, out, plan=plan)
+        plan.close()
+        assert_parity(got, gold, spmm_k_eff(s_arr), f"d={d} {out} {mask.H}x{mask.W}")
+
+    rng = np.random.default_rng(50 + d)
+    counts = 1 + np.arange(20) % 9
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    indices = np.concatenate([np.sort(rng.choice(20, n, replace=False)) for n in counts]).astype(np.int32)
+    check(with_values(W.BsrArrays(640, 640, 32, 32, indptr, indices, None), "RAND", seed=d), 8)
+    many = 32 * 700  # 700 stripes: more than the compute units
+    check(with_values(W.random_positions(many, 1024, 32, 32, 1500, rng), "RAND", seed=d), 8 if d == 32 else 4)
+    check(with_values(W.fill_row(64, 32 * 700, 32, 32, 1 + 700), "RAND", seed=3), 8)
+
+
+@pytest.mark.parametrize("out", ["f32", "bf16"])
+@pytest.mark.parametrize("offset,pad", [(0, 8), (1, 8), (2, 0), (4, 3)])
+def test_fused_attention_output_alignment(out, offset, pad):
+    """O at every element alignment and odd leading dimensions: the same bits
+    as aligned, and nothing written beside it."""
+    import torch
+    w = W.workload_attention(seq=1024, d=64)
+    mask, d = w["mask"], 64
+    want = run_attention(mask, w["q"], w["k"], w["v"], out)
+    dtype = torch.float32 if out == "f32" else torch.bfloat16
+    ld = d + pad
+    buf = torch.full((offset + mask.H * ld + 64,), 7.0, dtype=dtype, device="cuda")
+    o = buf[offset:offset + mask.H * ld].view(mask.H, ld)[:, :d]
+    dm, dq, dk, dv = (torch.from_numpy(np.ascontiguousarray(t).view(np.int16)).cuda()
+                      for t in (mask.data, w["q"], w["k"], w["v"]))
+    plan = capi.AttentionPlan(bsr_of(mask), d, out)
+    plan.run(dm, dq, dk, dv, o, stream=torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    plan.close()
+    np.testing.assert_array_equal(o.float().cpu().numpy(), want)
+    o.fill_(7.0)
+    assert bool((buf == 7.0).all())
