@@ -182,69 +182,127 @@ struct Tile {
         if constexpr (MF > SPAN) __builtin_amdgcn_sched_group_barrier(0x008, MF - SPAN, 0);
     }
 
-    // n steps of 64 (the last one 32 deep with `half_tail`); issue(k, stage)
-    // issues this wave's PER loads of step k, steps in ascending order.  A wave that is not `live`
+    // Products of the last k-step of a stage beside k-step 0's reads and the
+    // loads issue(k, into, 0 .. PER-1): one product, its share of the reads
+    // (over the first half of the products) and of the loads, and so on.  The
+    // loads in one burst between the barrier and the products held every wave
+    // at the same time while they issued: 8192^2, 128 x 128 blocks, 20%, K =
+    // 2048 76 -> 68 us; 8192^3, 256 x 256 blocks, 25% 238 -> 232 us (matrix
+    // cores busy 65% of the cycles, at the 1.77 GHz that the card holds there).
+    template <class Issue>
+    __device__ __forceinline__ void mul_read_issue(const Ops& o, int stage, Ops& next, int k, int into, Issue&& issue) {
+        constexpr int MF = FM * FN, RD = FM + (BK ? FN : 2 * FN);
+        constexpr int SPAN = MF > 1 ? MF / 2 : 1, PERM = (RD + SPAN - 1) / SPAN;
+        const uint8_t* st = smem + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < MF; ++i) {
+            f32x16& c = 3 % CH == 0 ? acc[i / FN][i % FN] : part[CH > 1 ? 3 % CH - 1 : 0][i / FN][i % FN];
+            c = mfma32(o.a[i / FN], o.b[i % FN], c);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int x = i * PERM; x < (i + 1) * PERM && x < RD; ++x) {
+                if (x < FM) {
+                    next.a[x] = *(const u32x4*)(st + a_rd[0] + x * 4096);
+                } else if constexpr (BK) {
+                    next.b[x - FM] = *(const u32x4*)(st + b_rd[0] + (x - FM) * 4096);
+                } else {
+                    const int nt = (x - FM) / 2, h = (x - FM) % 2;
+                    const u32x4 v = ld_tr_b16(st + b_rd[nt] + h * 8 * TN);
+                    next.b[nt][2 * h] = v.x;
+                    next.b[nt][2 * h + 1] = v.y;
+                }
+            }
+#pragma unroll
+            for (int j = i * PER / MF; j < (i + 1) * PER / MF; ++j) issue(k, into, j);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+
+    // n steps of 64 (the last one 32 deep with `half_tail`); issue(k, stage, j)
+    // issues load j of this wave's PER loads of step k, in ascending order.  A wave that is not `live`
     // (no output) loads and meets the barriers only.  Ends with every wave's
     // reads complete (the ring may be overwritten after a barrier).
     template <class Issue>
     __device__ __forceinline__ void run(int n, bool half_tail, bool live, Issue&& issue) {
 #pragma unroll
         for (int k = 0; k < S; ++k)
-            if (k < n) issue(k, k);
+            if (k < n)
+#pragma unroll
+                for (int j = 0; j < PER; ++j) issue(k, k, j);
         wait_stages<PER, S - 1>(min(S, n) - 1);  // step 0 landed
         barrier_no_fence();
         auto fence = [] { __builtin_amdgcn_sched_barrier(0); };
-        Ops o0, o1;
-        if (live) read(0, 0, o0);
-        fence();
-        int stage = 0;
-        for (int k = 0; k + 1 < n; ++k) {
-            if (live) {
-                mul(o0, 0);
-                read(stage, 1, o1);
-                interleave();
-                fence();
-                mul(o1, 1);
-                read(stage, 2, o0);
-                interleave();
-                fence();
-                mul(o0, 2);
-                read(stage, 3, o1);
-                interleave();
-                fence();
-            }
+        int stage = 0, k = 0;
+        // Step k+1 landed (k+2 .. k+S-1 in flight), and every wave has read step k.
+        auto sync_full = [&] {
             wait_lgkm0();
-            if (k + S < n)
-                wait_vmcnt<PER * (S - 2)>();  // step k+1 landed; k+2 .. k+S-1 in flight
-            else
-                wait_stages<PER, S - 2>(n - 2 - k);
+            wait_vmcnt<PER * (S - 2)>();
             barrier_no_fence();
-            if (k + S < n) issue(k + S, stage);
-            stage = stage == S - 1 ? 0 : stage + 1;
-            if (live) {
-                mul(o1, 3);
-                read(stage, 0, o0);
-                interleave();
+        };
+        auto sync = [&] {
+            wait_lgkm0();
+            wait_stages<PER, S - 2>(n - 2 - k);
+            barrier_no_fence();
+        };
+        auto next = [&] { stage = stage == S - 1 ? 0 : stage + 1; };
+        if (!live) {
+            for (; k + S < n; ++k) {
+                sync_full();
+#pragma unroll
+                for (int j = 0; j < PER; ++j) issue(k + S, stage, j);
+                next();
             }
-            fence();
+            for (; k + 1 < n; ++k) sync();
+            return;
         }
-        if (live) {
+        Ops o0, o1;
+        read(0, 0, o0);
+        fence();
+        auto first = [&] {
             mul(o0, 0);
             read(stage, 1, o1);
             interleave();
             fence();
             mul(o1, 1);
-            if (!half_tail) {
-                read(stage, 2, o0);
-                fence();
-                mul(o0, 2);
-                read(stage, 3, o1);
-                interleave();
-                fence();
-                mul(o1, 3);
-            }
-            fold();
+            read(stage, 2, o0);
+            interleave();
+            fence();
+            mul(o0, 2);
+            read(stage, 3, o1);
+            interleave();
+            fence();
+        };
+        for (; k + S < n; ++k) {
+            first();
+            sync_full();
+            const int freed = stage;
+            next();
+            mul_read_issue(o1, stage, o0, k + S, freed, issue);
         }
+        for (; k + 1 < n; ++k) {
+            first();
+            sync();
+            next();
+            mul(o1, 3);
+            read(stage, 0, o0);
+            interleave();
+            fence();
+        }
+        mul(o0, 0);
+        read(stage, 1, o1);
+        interleave();
+        fence();
+        mul(o1, 1);
+        if (!half_tail) {
+            read(stage, 2, o0);
+            fence();
+            mul(o0, 2);
+            read(stage, 3, o1);
+            interleave();
+            fence();
+            mul(o1, 3);
+        }
+        fold();
         wait_lgkm0();
     }
 };
@@ -259,8 +317,8 @@ struct Tile {
 // and looped kernels load Y anew for every 32 rows.
 //
 // What bounds it: the largest tile, on full 256 x 256 blocks and long K, the
-// matrix cores at the clock they hold (8192^3, 25%: 2730 -> 255-270 us, 1.02-
-// 1.08 PFLOP/s); the small ones the latency of a step's loads, which several
+// matrix cores at the clock they hold (8192^3, 25%: 2730 -> 232 us, 1.19
+// PFLOP/s; four waves of 128 x 128, which read a third less LDS: 254); the small ones the latency of a step's loads, which several
 // workgroups of a compute unit hide in turn (4096^2, 32 x 32 blocks, 25%,
 // K = 512: 34-41 -> 17-19 us; two stages and four workgroups beat four stages
 // and two, 19.6 : 22.3).  The 128 and 64-row tiles are for masks whose blocks
@@ -307,29 +365,32 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void sddmm_tile_kernel(SddmmTile
     const bool half_tail = (p.K & 63) != 0;
     const int64_t ystep = YT ? 128 : 128 * p.ldy;
     const int64_t xtwo = 32 * p.ldx, ytwo = (YT ? 32 : 2048 / TN) * p.ldy;  // bytes between loads j and j + 2
-    auto issue = [&](int k, int stage) {
-        if (half_tail && k == n - 1) {
+    auto issue = [&](int k, int stage, int j) {
+        const bool tail = half_tail && k == n - 1;
+        if (j == 0 && tail) {
             // The second half of the last step is past K: fetch its first
             // half twice (those products are not made).
 #pragma unroll
-            for (int j = 0; j < NPX; ++j)
-                if (t.kchunk(j, T::AL) >= 4) px[j] -= 64;
+            for (int i = 0; i < NPX; ++i)
+                if (t.kchunk(i, T::AL) >= 4) px[i] -= 64;
 #pragma unroll
-            for (int j = 0; j < NPY; ++j)
-                if (YT && t.kchunk(j, T::BL) >= 4) py[j] -= 64;
+            for (int i = 0; i < NPY; ++i)
+                if (YT && t.kchunk(i, T::BL) >= 4) py[i] -= 64;
         }
-#pragma unroll
-        for (int j = 0; j < T::AL; ++j) gl_lds16(px[j % 2] + (j / 2) * xtwo, t.a_lds(stage, j));
-#pragma unroll
-        for (int j = 0; j < T::BL; ++j) {
-            const uint8_t* src = py[j % 2] + (j / 2) * ytwo;
-            if (!YT && half_tail && k == n - 1 && t.nrow(j) >= 32) src -= 64 * p.ldy;
-            gl_lds16(src, t.b_lds(stage, j));
+        if (j < T::AL) {
+            gl_lds16(px[j % 2] + (j / 2) * xtwo, t.a_lds(stage, j));
+        } else {
+            const int jb = j - T::AL;
+            const uint8_t* src = py[jb % 2] + (jb / 2) * ytwo;
+            if (!YT && tail && t.nrow(jb) >= 32) src -= 64 * p.ldy;
+            gl_lds16(src, t.b_lds(stage, jb));
         }
+        if (j == T::PER - 1) {
 #pragma unroll
-        for (int j = 0; j < NPX; ++j) px[j] += 128;
+            for (int i = 0; i < NPX; ++i) px[i] += 128;
 #pragma unroll
-        for (int j = 0; j < NPY; ++j) py[j] += ystep;
+            for (int i = 0; i < NPY; ++i) py[i] += ystep;
+        }
     };
     const bool live = ((t.wc * T::FN * 32) >> cbs) < nc;
     t.run(n, half_tail, live, issue);
@@ -436,14 +497,17 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void spgemm_tile_kernel(SpgemmTi
         av[j] = 2u * (uint32_t)(t.krow(j, T::AL) * p.lda + 8 * t.kchunk(j, T::AL));
 #pragma unroll
     for (int j = 0; j < T::BL; ++j) bv[j] = 2u * (uint32_t)(t.nrow(j) * p.ldb + 8 * t.nchunk(j));
-    auto issue = [&](int k, int stage) {
-        if ((k & 63) == 0 && k > 0) fetch(k);
-        const uint16_t* a = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(lo, k & 63) * 32;
-        const uint16_t* b = p.b + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k & 63) * 32;
-#pragma unroll
-        for (int j = 0; j < T::AL; ++j) gl_lds16_s(av[j], a, t.a_lds(stage, j));
-#pragma unroll
-        for (int j = 0; j < T::BL; ++j) gl_lds16_s(bv[j], b, t.b_lds(stage, j));
+    const uint16_t *a = nullptr, *b = nullptr;  // the term's blocks
+    auto issue = [&](int k, int stage, int j) {
+        if (j == 0) {
+            if ((k & 63) == 0 && k > 0) fetch(k);
+            a = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(lo, k & 63) * 32;
+            b = p.b + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k & 63) * 32;
+        }
+        if (j < T::AL)
+            gl_lds16_s(av[j], a, t.a_lds(stage, j));
+        else
+            gl_lds16_s(bv[j - T::AL], b, t.b_lds(stage, j - T::AL));
     };
     t.run(n, false, true, issue);
 #pragma unroll
