@@ -2594,9 +2594,21 @@ static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_spli
                 launched = true;
             }
         }
-        if (!launched) {
-            if (pair) BSP_WIDE(8, true);
-            else BSP_WIDE(8, false);
+        // Entry pairs of two- and eight-stripe groups at the default ring run
+        // spmm_tile_kernel (both sides measured there), except in the
+        // instrumented build, whose switches it does not have.
+#ifdef BSP_TIMELINE
+        constexpr bool tiles = false;
+#else
+        constexpr bool tiles = (G == 8 && S == 4) || G == 2;
+#endif
+        if (!launched && pair) {
+            if constexpr (tiles)
+                launch_spmm_tile(a, G, out_bf16, grid, stream);
+            else
+                BSP_WIDE(8, true);
+        } else if (!launched) {
+            BSP_WIDE(8, false);
         }
 #undef BSP_WIDE
     } else {

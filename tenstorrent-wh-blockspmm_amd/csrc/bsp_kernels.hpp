@@ -283,6 +283,9 @@ inline SpmmVariant spmm_default_variant(int tile_n, int group) {
     }
 }
 
+// SpMM over row groups of 2 or 8 stripes with 256-column tiles by
+// spmm_tile_kernel (C a multiple of 64).
+void launch_spmm_tile(const SpmmArgs& a, int group, bool out_bf16, int grid, hipStream_t stream);
 // Launches the SpMM kernel and, when the plan has split rows, the reduce kernel.
 hipError_t launch_spmm(const SpmmArgs& a, const SpmmVariant& v, bool out_bf16, int grid, int n_split,
                        hipStream_t stream);

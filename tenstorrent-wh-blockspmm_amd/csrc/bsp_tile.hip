@@ -1,5 +1,5 @@
-// Tile kernels: SDDMM over long K and SpGEMM over blocks of 64 and more, each
-// a workgroup computing a TM x TN output tile (gfx950).
+// Tile kernels: SDDMM over long K, SpGEMM over blocks of 64 and more and SpMM
+// over row groups, each a workgroup computing a TM x TN output tile (gfx950).
 //
 // Both are a product of an A panel, TM rows contiguous along k (X rows, rows
 // of an A block), and a B panel of TN columns, along k in steps of 64.  A step
@@ -21,7 +21,7 @@
 // step, and no part of a step is reads alone.
 //
 // Reference semantics: sparse_common/bsr_matrix.hpp:816-857 (SDDMM), :741-810
-// (SpGEMM).
+// (SpGEMM); block_spmm/inc/bsr_matrix.hpp:954-1000 (SpMM).
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -526,6 +526,98 @@ __global__ __launch_bounds__(64 * WR * WC, WPE) void spgemm_tile_kernel(SpgemmTi
 }
 
 // ---------------------------------------------------------------------------
+// SpMM over row groups of RW stripes with a 256-column tile: the work items of
+// spmm_group_wide_kernel where C is a multiple of 64 (an item's entries are then
+// pairs, the two 32-column halves of 64 columns of a block), a pair a step: half
+// the barriers, and the loads between the products.  Each output adds the same
+// products in the same order (the results are bit-identical).
+//
+// What bounds it: at RW = 8 (one workgroup per compute unit) the matrix cores at
+// the clock they hold, and L2 fills; at RW = 2 (two) the fills, B's panel per 64
+// rows.  us of spmm_group_wide_kernel : this one, 8192^3: 256 x 256 blocks 25%
+// 256 : 244 (f32 out 267 : 247), 50% 460 : 428; 64 x 64 blocks 25% 488 : 356;
+// 256 x 64 blocks, 8192^2 10%, N = 4096 64.3 : 60.4.  Short rows gain nothing
+// (16384 x 4096, 6% of 256 x 256, N = 2048 39.8 : 39.7; 8192 x 6144, 10% of 64 x
+// 64, N = 2048 33.5 : 33.5).  RW = 4 is left to spmm_group_wide_kernel, whose
+// smaller stages let two workgroups share a compute unit (8192 x 6144, 10% of
+// 128 x 64, N = 2048 29 there, 34 here with two or three stages; 4096^3 25% of
+// 128 x 128 41 : 46; only at 8192^3 three stages win, 290 : 281).
+template <int RW, int S, bool OUT_BF16, int WPE>
+__global__ __launch_bounds__(512, WPE) void spmm_tile_kernel(SpmmArgs p) {
+    using namespace tile_detail;
+    using T = Tile<32 * RW, 256, 2, 4, S, false>;
+    __shared__ __attribute__((aligned(1024))) uint8_t smem[T::LDS];
+    const SpmmWg it = load_const(p.wgs + blockIdx.x);
+    if (it.row < 0) return;  // idle slot (uniform)
+    T t(smem);
+    const int n = (it.e_end - it.e_begin) >> 1;  // steps
+    // Words of steps 64c .. 64c+63 in lanes (a pair's first entry names both).
+    const int64_t* ents = p.ents + it.e_begin;
+    uint32_t lo = 0, hi = 0;
+    auto fetch = [&](int base) {
+        if (base + t.lane < n) {
+            const int64_t w = ents[2 * (int64_t)(base + t.lane)];
+            lo = (uint32_t)w;
+            hi = (uint32_t)((uint64_t)w >> 32);
+        }
+        __asm__ volatile("" : "+v"(lo), "+v"(hi));
+    };
+    fetch(0);
+    // Byte offsets within the block's panel, and from the first of the eight
+    // rows of B that this wave loads (ldb < 2^26: below 4 GB).
+    static_assert(T::BL * 1024 == 8 * 2 * 256, "eight rows of B per wave and step");
+    uint32_t av[T::AL], bv[T::BL];
+#pragma unroll
+    for (int j = 0; j < T::AL; ++j)
+        av[j] = 2u * (uint32_t)(t.krow(j, T::AL) * p.lda + 8 * t.kchunk(j, T::AL));
+#pragma unroll
+    for (int j = 0; j < T::BL; ++j)
+        bv[j] = (uint32_t)(2 * ((int64_t)(t.nrow(j) - 8 * t.wave) * p.ldb + 8 * t.nchunk(j)));
+    const uint16_t* bw = p.b + (int64_t)(8 * t.wave) * p.ldb + (int64_t)it.tile * 256;
+    const uint16_t *a = nullptr, *b = nullptr;  // the step's panels
+    auto issue = [&](int k, int stage, int j) {
+        if (j == 0) {
+            if ((k & 63) == 0 && k > 0) fetch(k);
+            a = p.a + (int64_t)(uint32_t)__builtin_amdgcn_readlane(hi, k & 63) * 32;
+            b = bw + (int64_t)(uint32_t)__builtin_amdgcn_readlane(lo, k & 63) * p.ldb;
+        }
+        if (j < T::AL)
+            gl_lds16_s(av[j], a, t.a_lds(stage, j));
+        else
+            gl_lds16_s(bv[j - T::AL], b, t.b_lds(stage, j - T::AL));
+    };
+    if (n > 0) t.run(n, false, true, issue);
+#pragma unroll
+    for (int i = 0; i < T::FM; ++i) {
+        const int st = t.wr * T::FM + i;  // stripe within the group
+        if (it.slot >= 0) {
+            // A piece of a split group: stripe st's partial in its own slot
+            // (32-column tile c's column l at ((c % 2) * 16 + v) * 256 + (c / 2) * 64 + l).
+            const int slot = it.base + st * it.npieces + (it.slot - it.base);
+            float* mine = p.ws + ((int64_t)slot * p.n_tiles + it.tile) * (2 * 16 * 256);
+#pragma unroll
+            for (int nt = 0; nt < T::FN; ++nt) {
+                const int c = t.wc * T::FN + nt;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) mine[((c & 1) * 16 + v) * 256 + (c >> 1) * 64 + t.lane] = t.acc[i][nt][v];
+            }
+            continue;
+        }
+#pragma unroll
+        for (int nt = 0; nt < T::FN; ++nt)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int64_t row = (int64_t)(it.row + st) * 32 + 8 * (v >> 2) + 4 * t.q + (v & 3);
+                const int64_t idx = row * p.ldc + (int64_t)it.tile * 256 + (t.wc * T::FN + nt) * 32 + t.l32;
+                if (OUT_BF16)
+                    store_out(&((uint16_t*)p.c)[idx], f32_to_bf16_rne(t.acc[i][nt][v]));
+                else
+                    store_out(&((float*)p.c)[idx], t.acc[i][nt][v]);
+            }
+    }
+}
+
+// ---------------------------------------------------------------------------
 template <int TM, int TN, int WR, int WC, int S, int CH, int WPE>
 static void launch_sddmm_tile_t(const SddmmTileArgs& a, bool y_colmajor, bool out_bf16, int grid, hipStream_t stream) {
     const dim3 g(grid), b(64 * WR * WC);
@@ -572,6 +664,21 @@ hipError_t launch_spgemm_tile(const SpgemmTileArgs& a, int tile, bool out_bf16, 
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+template <int RW, int S, int WPE>
+static void launch_spmm_tile_t(const SpmmArgs& a, bool out_bf16, int grid, hipStream_t stream) {
+    if (out_bf16)
+        hipLaunchKernelGGL((spmm_tile_kernel<RW, S, true, WPE>), dim3(grid), dim3(512), 0, stream, a);
+    else
+        hipLaunchKernelGGL((spmm_tile_kernel<RW, S, false, WPE>), dim3(grid), dim3(512), 0, stream, a);
+}
+
+void launch_spmm_tile(const SpmmArgs& a, int group, bool out_bf16, int grid, hipStream_t stream) {
+    if (group == 2)
+        launch_spmm_tile_t<2, 2, 4>(a, out_bf16, grid, stream);
+    else
+        launch_spmm_tile_t<8, 2, 2>(a, out_bf16, grid, stream);
 }
 
 }  // namespace bsp

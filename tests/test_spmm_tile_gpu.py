@@ -1,0 +1,51 @@
+"""The 256-column SpMM tile kernel (row groups of two and eight stripes, C a
+multiple of 64) on the GPU against the oracle where its steps can go wrong: one
+step an item, rows longer than its 64-step word chunk, empty block rows, pieces
+of split rows, B and C wider than N.
+
+Bound: both sides add the same n products (exact in fp32) of values in [-1, 1]
+in fp32 in different orders: each is off by at most n^2 * 2^-24; twice that is
+allowed, and one bf16 rounding (2^-8) on bf16 output."""
+import numpy as np
+import pytest
+
+from helpers import W, bsr_of, capi, golden_spmm, spmm_k_eff, strided_run, with_values
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("out_dtype", ["f32", "bf16"])
+@pytest.mark.parametrize("split", [0, 6])
+@pytest.mark.parametrize("R,C,Wd,counts", [
+    (64, 64, 4544, [1, 0, 71, 64, 2]),      # steps of different blocks; 65 and more, empty, one
+    (64, 192, 1344, [7, 0, 1]),             # three steps a block
+    (128, 64, 640, [3, 0, 10]),             # eight-stripe groups need R = 256: two-stripe ones of R = 128
+    (256, 64, 4288, [67, 0, 1]),
+    (256, 128, 1024, [2, 8, 0]),
+])
+def test_tile_edges(R, C, Wd, counts, split, out_dtype, monkeypatch):
+    group = 8 if R == 256 else 2
+    monkeypatch.setenv("BSP_SPMM_GROUP", str(group))
+    monkeypatch.setenv("BSP_SPMM_WIDE_GROUP", "2")
+    monkeypatch.setenv("BSP_SPMM_SPLIT", str(split or 100000))
+    rng = np.random.default_rng(R + C)
+    indptr = np.concatenate([[0], np.cumsum(counts)]).astype(np.int32)
+    cols = np.concatenate([np.sort(rng.choice(Wd // C, n, replace=False)) for n in counts]).astype(np.int32)
+    a = with_values(W.BsrArrays(R * len(counts), Wd, R, C, indptr, cols), "RAND", seed=R + C)
+    N = 512
+    b = W.dense_content(Wd, N, "RAND", rng)
+    plan = capi.SpmmPlan(bsr_of(a), N, out_dtype)
+    info = plan.info()
+    assert (info["group"], info["tile_n"]) == (group, 256) and (info["n_split_rows"] > 0) == bool(split), info
+    import torch
+    print(R, C, split, out_dtype, flush=True)
+    got, after, before = strided_run(
+        a, b, out_dtype, N + 24, N + 32,
+        lambda da, bw, cw: plan.run(da, bw, cw, stream=torch.cuda.current_stream().cuda_stream))
+    plan.close()
+    np.testing.assert_array_equal(after.view(np.uint8), before.view(np.uint8), err_msg="C's padding was written")
+    gold = golden_spmm(a, b)
+    n = spmm_k_eff(a).astype(np.float64)
+    bound = 2 * (n * n + 1) * 2.0 ** -24 + (2.0 ** -8 * np.abs(gold) if out_dtype == "bf16" else 0)
+    err = np.abs(got.astype(np.float64) - gold)
+    assert np.isfinite(got).all() and np.all(err <= bound), err.max()
