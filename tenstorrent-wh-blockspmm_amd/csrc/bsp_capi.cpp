@@ -795,8 +795,12 @@ int bsp_sddmm_plan_create(bsp_plan** out, const bsp_bsr_desc* mask, int64_t K, i
     int cus = 256;
     st = device_cus(device, &cus);
     if (st != BSP_OK) return st;
+#ifdef BSP_TIMELINE
+    const bsp::SddmmTileVariant tv{};  // (the tile kernel has no switches to leave work out)
+#else
     const bsp::SddmmTileVariant tv =
         std::getenv("BSP_SDDMM_LOOP") ? bsp::SddmmTileVariant{} : bsp::sddmm_choose_tile(mask, K, cus);
+#endif
     const int tile_m = tv.tile_m;
     bsp::SddmmSchedule s;
     bsp::SddmmTiles ts;
@@ -858,8 +862,6 @@ int bsp_sddmm(const bsp_plan* p, const uint16_t* mask_vals, const uint16_t* x, i
     DeviceGuard g(p->device);
     if (g.err != hipSuccess) return hip_fail(g.err, "hipSetDevice");
     if (p->tile) {
-        if (launch_skips() != 0)
-            return fail(BSP_ERR_UNSUPPORTED, "this plan's kernel has no switches to leave work out");
         bsp::SddmmTileArgs ta{};
         ta.mask = mask_vals;
         ta.x = x;
