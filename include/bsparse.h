@@ -103,10 +103,12 @@ typedef struct bsp_plan_info {
     int32_t grid;        /* workgroups per launch */
     int32_t max_item_entries;
     int32_t stages;      /* SpMM, SpGEMM: depth of the LDS ring (entries in
-                            flight + 1); SDDMM: 1 = one-shot kernel, 0 = looped */
+                            flight + 1); SDDMM: 1 = one-shot kernel, 0 = looped,
+                            more = the tile kernel's ring; attention: 1 */
     int32_t group;       /* SpMM: 32-row stripes of one block row per workgroup
-                            (1; or 2, 4, 8 for blocks of R >= 64) */
-    int32_t waves;       /* SpMM: waves per workgroup (fixed at plan creation) */
+                            (1; or 2, 4, 8 for blocks of R >= 64); SDDMM and
+                            SpGEMM tile kernels: stripes of a tile */
+    int32_t waves;       /* SpMM, attention: waves per workgroup (fixed at plan creation) */
     int64_t workspace_bytes; /* device scratch owned by the plan */
     int32_t persistent;  /* SpMM: 0 = one work item per workgroup; 1 or 2 =
                             persistent kernel with that many pipelines per
