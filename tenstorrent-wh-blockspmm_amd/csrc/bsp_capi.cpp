@@ -43,6 +43,7 @@ struct bsp_plan {
     int32_t tile = 0;            // SDDMM, SpGEMM: the tile kernel runs this plan on tiles of that height
     bsp::SddmmTileVariant sddmm_tile{};
     int32_t narrow = 0;          // SpMM of fewer than 128 columns: waves of spmm_narrow_kernel
+    int32_t group_tile = 0;      // SpMM row groups: spmm_tile_kernel runs this plan
     int32_t cb_shift = 0;        // SDDMM tiles: log2 of the column chunks' width
     // SpMM persistent kernel: variant, unit records and A words (the B words
     // go in d_ent_off, the workgroup heads in d_wgs; d_apw with stripe pairs).
@@ -616,6 +617,16 @@ int make_spmm_plan(bsp_plan** out, int kind, const bsp_bsr_desc* a, int64_t N, i
         p->narrow = N == 32 || items <= cus ? 8 : N == 96 && entries < 8 * items ? 0 : 4;
         if (p->narrow) p->info.waves = p->narrow;
     }
+#ifndef BSP_TIMELINE
+    // Eight-stripe groups at the default ring always; two-stripe ones from four
+    // 64-deep steps a block row on average, below which a tile's two stages
+    // are barely used (64 x 64 blocks, 8192^2, N = 2048: 2.5 steps 20.1 us by the
+    // wide kernel, 20.9 by this one; 9.6 steps, 6144 wide, 33.1 : 32.7).  (Not in
+    // the instrumented build, whose switches spmm_tile_kernel does not have.)
+    if (s.tile_n == 256 && p->info.waves == 8 && a->C % 64 == 0)
+        p->group_tile = (s.group == 8 && p->info.stages == 4) ||
+                        (s.group == 2 && a->nblocks * (a->C / 64) >= 4 * (a->H / a->R));
+#endif
     if (kind == 3) {
         p->info.kind = 3;
         p->info.stages = 1;
@@ -728,7 +739,7 @@ int bsp_spmm(const bsp_plan* p, const uint16_t* a_vals, const uint16_t* b, int64
         e = bsp::launch_spmm_stream(sa, p->stream_variant, p->out_dtype == BSP_DTYPE_BF16, p->info.grid,
                                     (hipStream_t)stream);
     } else {
-        const bsp::SpmmVariant v{p->info.tile_n, p->info.stages, p->info.group, p->info.waves, p->narrow};
+        const bsp::SpmmVariant v{p->info.tile_n, p->info.stages, p->info.group, p->info.waves, p->narrow, p->group_tile};
         e = bsp::launch_spmm(args, v, p->out_dtype == BSP_DTYPE_BF16, p->info.grid, p->info.n_split_rows,
                              (hipStream_t)stream);
     }

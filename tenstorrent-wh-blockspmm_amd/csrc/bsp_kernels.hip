@@ -2560,7 +2560,7 @@ static void launch_spmm_narrow(const SpmmArgs& a, int waves, bool out_bf16, int 
 }
 
 template <int NTW, int S, int G>
-static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_split, int waves, int narrow,
+static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_split, int waves, int narrow, int tile,
                           hipStream_t stream) {
     if constexpr (G == 1) {
         if (narrow)
@@ -2594,21 +2594,20 @@ static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_spli
                 launched = true;
             }
         }
-        // Entry pairs of two- and eight-stripe groups at the default ring run
-        // spmm_tile_kernel (both sides measured there), except in the
-        // instrumented build, whose switches it does not have.
-#ifdef BSP_TIMELINE
-        constexpr bool tiles = false;
-#else
-        constexpr bool tiles = (G == 8 && S == 4) || G == 2;
-#endif
-        if (!launched && pair) {
-            if constexpr (tiles)
-                launch_spmm_tile(a, G, out_bf16, grid, stream);
-            else
-                BSP_WIDE(8, true);
+        if (!launched && tile) {
+            launch_spmm_tile(a, G, out_bf16, grid, stream);
         } else if (!launched) {
-            BSP_WIDE(8, false);
+            // (Eight stripes in entry pairs at the default ring always run
+            // spmm_tile_kernel, but for the instrumented build.)
+#ifdef BSP_TIMELINE
+            constexpr bool wide_pair = true;
+#else
+            constexpr bool wide_pair = G != 8 || S != 4;
+#endif
+            if constexpr (wide_pair) {
+                if (pair) BSP_WIDE(8, true);
+            }
+            if (!pair) BSP_WIDE(8, false);
         }
 #undef BSP_WIDE
     } else {
@@ -2629,11 +2628,12 @@ static void launch_spmm_t(const SpmmArgs& a, bool out_bf16, int grid, int n_spli
 hipError_t launch_spmm(const SpmmArgs& a, const SpmmVariant& v, bool out_bf16, int grid, int n_split,
                        hipStream_t stream) {
     if (grid <= 0) return hipSuccess;
-    if (!spmm_variant_supported(v) || (v.narrow && (v.tile_n != 128 || v.group != 1 || a.N >= 128)))
+    if (!spmm_variant_supported(v) || (v.narrow && (v.tile_n != 128 || v.group != 1 || a.N >= 128)) ||
+        (v.tile && (v.tile_n != 256 || (v.group != 2 && v.group != 8) || v.waves != 8 || a.lda % 64)))
         return hipErrorInvalidValue;
 #define BSP_SPMM_CASE(TN, S, G)                                                   \
     if (v.tile_n == TN && v.stages == S && v.group == G) {                       \
-        launch_spmm_t<TN / 128, S, G>(a, out_bf16, grid, n_split, v.waves, v.narrow, stream); \
+        launch_spmm_t<TN / 128, S, G>(a, out_bf16, grid, n_split, v.waves, v.narrow, v.tile, stream); \
         return hipGetLastError();                                                \
     }
     BSP_SPMM_VARIANTS(BSP_SPMM_CASE)

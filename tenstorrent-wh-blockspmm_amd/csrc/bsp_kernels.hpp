@@ -263,6 +263,7 @@ struct SpmmVariant {
     int group;
     int waves = 4;   // 256-column row groups: 8 (default) or 4 waves per workgroup
     int narrow = 0;  // N < 128, single stripes: spmm_narrow_kernel with that many waves (4 or 8; 0: spmm_kernel)
+    int tile = 0;    // 256-column row groups of 2 or 8, eight waves, C a multiple of 64: spmm_tile_kernel
 };
 
 inline bool spmm_variant_supported(const SpmmVariant& v) {

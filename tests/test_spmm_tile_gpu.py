@@ -19,7 +19,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("R,C,Wd,counts", [
     (64, 64, 4544, [1, 0, 71, 64, 2]),      # steps of different blocks; 65 and more, empty, one
     (64, 192, 1344, [7, 0, 1]),             # three steps a block
-    (128, 64, 640, [3, 0, 10]),             # eight-stripe groups need R = 256: two-stripe ones of R = 128
+    (128, 64, 640, [3, 0, 10]),             # two-stripe groups of R = 128
     (256, 64, 4288, [67, 0, 1]),
     (256, 128, 1024, [2, 8, 0]),
 ])
